@@ -787,6 +787,18 @@ int mirl_grpo_advantage(const int64_t* prompts, int64_t B, int64_t K,
                         int normalize, float* adv, float* baseline, float* std,
                         uint8_t* trivial, void* stream);
 
+/* mirl_grpo_advantage with a workspace of
+ * mirl_grpo_advantage_workspace_bytes(B, K) bytes (8-byte aligned; 0 and NULL for
+ * K == 1): rows are grouped by a hash confirmed by one full comparison each
+ * instead of being compared pair by pair.  Same results. */
+int64_t mirl_grpo_advantage_workspace_bytes(int64_t B, int64_t K);
+int mirl_grpo_advantage_ws(const int64_t* prompts, int64_t B, int64_t K,
+                           int64_t prompt_stride, const float* rewards,
+                           const float* std_rewards, const float* valid_mask,
+                           int leave_one_out,
+                           int normalize, float* adv, float* baseline, float* std,
+                           uint8_t* trivial, void* workspace, void* stream);
+
 /* ---------------------------------------------------------------------- */
 /* Packed-sequence glue                                                    */
 /* ---------------------------------------------------------------------- */

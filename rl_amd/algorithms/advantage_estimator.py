@@ -1,7 +1,7 @@
 """GRPO advantage estimator: drop-in for the GRPO part of ``nemo_rl.algorithms.advantage_estimator``.
 
 ``GRPOAdvantageEstimator.compute_advantage`` runs the group-statistics kernel
-(one thread per sample) and returns the advantages broadcast to the token mask
+(one wave per sample) and returns the advantages broadcast to the token mask
 shape, as the reference does (reference advantage_estimator.py:94-145).
 """
 
