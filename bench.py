@@ -58,7 +58,7 @@ sys.path.insert(0, str(ROOT))
 METRIC = "logprob+PG-loss fwd/bwd tokens/s and HBM GB/s (% peak) at V=151936 bf16"
 PEAK_HBM_GBPS = 8000.0
 PEAK_BF16_TFLOPS = 2500.0  # dense bf16 MFMA (fp16 the same)
-PEAK_FP32_TFLOPS = 157.3  # dense fp32 MFMA
+PEAK_FP32_TFLOPS = PEAK_BF16_TFLOPS / 6  # fp32 products as six bf16 products each
 
 
 def parse():

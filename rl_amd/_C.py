@@ -1290,7 +1290,8 @@ def gemm_bf16_abt(a: torch.Tensor, b: torch.Tensor, k: int, out: torch.Tensor, k
 def gemm_f32_abt(a: torch.Tensor, b: torch.Tensor, k: int, out: torch.Tensor, k_splits: int = 1,
                  accumulate: bool = False, count: Optional[torch.Tensor] = None,
                  count_off: int = 0, count_axis: int = COUNT_ROWS) -> None:
-    """out = a[:, :k] . b[:, :k]^T in fp32 on the MFMA units (fp32 MFMA).
+    """out = a[:, :k] . b[:, :k]^T in fp32 on the MFMA units (each operand as three bf16
+    planes that add up to it exactly, six products of planes into fp32 accumulators).
 
     a [M, >=k], b [N, >=k] fp32 (unit stride, row strides multiples of 4 elements,
     16-byte aligned, k a multiple of 64); out fp32 [M, N] (out = or +=), or

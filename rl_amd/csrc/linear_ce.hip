@@ -32,6 +32,7 @@
 // is C[(v / 4) * 8 + (l / 32) * 4 + v % 4][l % 32].
 
 #include <type_traits>
+#include <utility>
 
 #include "common.h"
 
@@ -60,7 +61,8 @@ struct Mma<F16> {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
   }
 };
-// fp32 operands (plain GEMM only): a 16-byte fragment holds four hidden
+// fp32 operands (plain GEMM only), for tiles that the bf16 planes do not cover
+// (see the kernel): a 16-byte fragment holds four hidden
 // elements of a row, k = (l / 32) * 4 + 0..3, and feeds four
 // v_mfma_f32_32x32x2_f32, element e of both fragments to the e-th one.  That
 // instruction takes A[l % 32][l / 32] and B[l / 32][l % 32] from lane l, so the
@@ -135,6 +137,36 @@ template <int N>
 __device__ __forceinline__ void wait_vm_barrier() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// The low bf16 of a pair, widened.  By a byte permute: for a shift, the compiler would
+// form the low half once more with a conversion of its own.
+__device__ __forceinline__ float low_bf16(uint32_t w) {
+  return __uint_as_float(__builtin_amdgcn_perm(0u, w, 0x01000c0cu));
+}
+
+// Per 16-bit half of w: 2 w - 1, and the smaller of two.  In asm: taken apart into
+// halves, the compiler converts and permutes each pair again.
+__device__ __forceinline__ uint32_t twice_less_one(uint32_t w) {
+  uint32_t r;
+  asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(r) : "v"(w), "v"(0x00020002u), "v"(0xffffffffu));
+  return r;
+}
+__device__ __forceinline__ uint32_t min_u16x2(uint32_t a, uint32_t b) {
+  uint32_t r;
+  asm("v_pk_min_u16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+// f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>): a loop whose index
+// the body may use in a constant expression.
+template <int... I, class F>
+__device__ __forceinline__ void static_for_(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_(std::make_integer_sequence<int, N>{}, f);
 }
 
 enum LceMode { kFwd = 0, kGrad = 1, kGemm = 2 };
@@ -390,15 +422,10 @@ void lce_tile_kernel(LceParams P) {
 
   constexpr int kL = 2 * kDmaPerWave;  // direct loads per wave and stage
   static_assert(kL == kTM * kTN, "one direct load per MFMA of block 3");
-  // Prologue: stage data 0 and 1 in flight; wait for 0 and read its block-0 fragments.
-#pragma unroll
-  for (int q = 0; q < kL; ++q) dma(st0, 0, q);
-#pragma unroll
-  for (int q = 0; q < kL; ++q) dma(st1, 1, q);
-  wait_vm_barrier<kL>();
-#pragma unroll
-  for (int idx = 0; idx < kTM + kTN; ++idx) fread(0, st0, 0, idx);
-
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, 1>;
+  using T_ = std::integral_constant<bool, true>;
+  using F_ = std::integral_constant<bool, false>;
   // One stage t (S = t % 2): four MFMA blocks kk = 0..3 of 16 MFMAs (16 hidden
   // elements each for 16-bit operands; for fp32, 8 elements in four instructions).  While block kk runs on fragment set kk % 2, block kk + 1's
   // fragments are read into the other set.  Before block 3 this wave waits for
@@ -434,17 +461,176 @@ void lce_tile_kernel(LceParams P) {
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  using S0 = std::integral_constant<int, 0>;
-  using S1 = std::integral_constant<int, 1>;
-  using T_ = std::integral_constant<bool, true>;
-  using F_ = std::integral_constant<bool, false>;
-  int t = 0;
-  for (; t < nst - kStages; t += kStages) {
-    step(t, S0{}, T_{}, T_{});
-    step(t + 1, S1{}, T_{}, T_{});
+  auto run_stages = [&]() __attribute__((always_inline)) {
+    // Prologue: stage data 0 and 1 in flight; wait for 0 and read its block-0 fragments.
+#pragma unroll
+    for (int q = 0; q < kL; ++q) dma(st0, 0, q);
+#pragma unroll
+    for (int q = 0; q < kL; ++q) dma(st1, 1, q);
+    wait_vm_barrier<kL>();
+#pragma unroll
+    for (int idx = 0; idx < kTM + kTN; ++idx) fread(0, st0, 0, idx);
+    int t = 0;
+    for (; t < nst - kStages; t += kStages) {
+      step(t, S0{}, T_{}, T_{});
+      step(t + 1, S1{}, T_{}, T_{});
+    }
+    step(t, S0{}, T_{}, F_{});
+    step(t + 1, S1{}, F_{}, F_{});
+  };
+
+  if constexpr (std::is_same<E, F32>::value) {
+    // ---- fp32 operands as three bf16 planes each ----
+    //
+    // x = x0 + x1 + x2 exactly, with x0 = bf16(x), x1 = bf16(x - x0) and
+    // x2 = x - x0 - x1 (at most eight significant bits are left), so a product of
+    // two elements is the sum of nine bf16 products; the three below 2^-25 of it
+    // (a1 b2, a2 b1, a2 b2) are left out and the six others summed into the same
+    // fp32 accumulators, the small ones first.  The fp32 MFMA runs at 1/16 of the
+    // bf16 rate, so six bf16 products cost 3/8 of one fp32 product, and 32 k-terms
+    // enter an accumulator in 12 roundings instead of 16: [2048, 4096] x
+    // [65536, 4096]^T 149 -> 237 TFLOP/s (1420 of bf16), error against 64 bits 1.14e-6
+    // -> 1.01e-6 of the result (K = 64: 1.46e-7 -> 1.09e-7).  Bound by the clock: the
+    // MFMA units are busy 87% of the cycles, at 1.5 GHz under this load.
+    //
+    // Each lane reads the fp32 fragments of the coming 16 hidden elements and
+    // splits them while the 96 MFMAs of the current ones run: 52 VALU
+    // instructions per fragment, five in the shadow of each MFMA.  (Residuals by
+    // v_dot2_f32_bf16, 28 instructions, were slower: 207 TFLOP/s.)
+    using frag16 = typename Mma<BF16>::frag;
+    constexpr int kPl = 3, kFr = kTM + kTN;
+    constexpr int kOpSlots = 11;  // slots a fragment's split takes
+    constexpr int kSlots = 2 * kPl * kTM * kTN;      // MFMAs per 16 hidden elements
+    constexpr int kOps = 52, kPer = 5;               // VALU ops per fragment, per slot
+    constexpr int kFirst = kSlots - kFr * kOpSlots;  // slot of the first split op
+    static_assert(kFirst >= 4 && kKK == 4, "reads ahead of the split");
+    // the lane's 8 hidden elements 16 kk + 8 (lane / 32) + 0..7 of a row: two chunks
+    int foff[2][2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) foff[kk][c] = lds_off(frow, kk * 4 + (lane >> 5) * 2 + c);
+    frag16 pl[2][kFr][kPl];  // [set][A fragments, then B][plane]
+    float raw[3][8];
+    float h0, h1, r0, r1;
+    // the least nonzero magnitude of a first plane, as 2 |bits| - 1 (zero: 65535)
+    uint32_t mag, least = 0xffffffffu;
+    uint32_t out[kPl][4];
+    auto read_raw = [&](const unsigned char* stage, int kk, int f) __attribute__((always_inline)) {
+      const unsigned char* rows = f < kTM ? stage + (wm * kWM + f * 32) * kRowBytes
+                                          : stage + kHalfBytes + (wn * kWN + (f - kTM) * 32) * kRowBytes;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const frag q = *reinterpret_cast<const frag*>(rows + foff[kk][c]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) raw[f % 3][c * 4 + e] = q[e];
+      }
+    };
+    // op N of the split of fragment F into set SET
+    auto split_op = [&](auto set_c, auto f_c, auto n_c) __attribute__((always_inline)) {
+      constexpr int F = decltype(f_c)::value, N = decltype(n_c)::value;
+      constexpr int P = N / 13, O = N % 13;
+      float* x = raw[F % 3];
+      if constexpr (O == 0) out[0][P] = BF16::pack2(x[2 * P], x[2 * P + 1]);
+      else if constexpr (O == 1) h0 = low_bf16(out[0][P]);
+      else if constexpr (O == 2) h1 = __uint_as_float(out[0][P] & 0xffff0000u);
+      else if constexpr (O == 3) r0 = x[2 * P] - h0;
+      else if constexpr (O == 4) r1 = x[2 * P + 1] - h1;
+      else if constexpr (O == 5) out[1][P] = BF16::pack2(r0, r1);
+      else if constexpr (O == 6) h0 = low_bf16(out[1][P]);
+      else if constexpr (O == 7) h1 = __uint_as_float(out[1][P] & 0xffff0000u);
+      else if constexpr (O == 8) r0 = r0 - h0;
+      else if constexpr (O == 9) r1 = r1 - h1;
+      else if constexpr (O == 10) out[2][P] = BF16::pack2(r0, r1);
+      else if constexpr (O == 11) mag = twice_less_one(out[0][P]);
+      else least = min_u16x2(least, mag);
+      if constexpr (N == kOps - 1) {
+#pragma unroll
+        for (int k = 0; k < kPl; ++k) {
+          const vu4 q = {out[k][0], out[k][1], out[k][2], out[k][3]};
+          pl[decltype(set_c)::value][F][k] = __builtin_bit_cast(frag16, q);
+        }
+      }
+    };
+    // One step: the 96 MFMAs of set SET (products a2 b0, a0 b2, a1 b1, a1 b0, a0 b1,
+    // a0 b0 of the 16 tiles), beside them the reads and the split of the next 16
+    // hidden elements (half kk of `stage`) into the other set, and with LOAD the
+    // direct loads of stage data t_load into `into`.
+    auto step16 = [&](auto set_c, const unsigned char* stage, int kk, auto load_c, unsigned char* into,
+                      int t_load) __attribute__((always_inline)) {
+      constexpr int SET = decltype(set_c)::value;
+      constexpr bool LOAD = decltype(load_c)::value;
+      static_for<kSlots>([&](auto q_c) __attribute__((always_inline)) {
+        constexpr int Q = decltype(q_c)::value;
+        constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+        constexpr int PR = Q / (kTM * kTN), I = Q / kTN % kTM, J = Q % kTN;
+        acc[I][J] = Mma<BF16>::run(pl[SET][I][pa[PR]], pl[SET][kTM + J][pb[PR]], acc[I][J]);
+        // the first two fragments are read at once, each other one a split ahead
+        if constexpr (Q == 0) read_raw(stage, kk, 0);
+        if constexpr (Q == 2) read_raw(stage, kk, 1);
+        if constexpr (Q >= kFirst) {
+          constexpr int F = (Q - kFirst) / kOpSlots, N = (Q - kFirst) % kOpSlots * kPer;
+          if constexpr (N == 0 && F + 2 < kFr) read_raw(stage, kk, F + 2);
+          static_for<kPer>([&](auto u_c) __attribute__((always_inline)) {
+            if constexpr (N + decltype(u_c)::value < kOps)
+              split_op(std::integral_constant<int, SET ^ 1>{}, std::integral_constant<int, F>{},
+                       std::integral_constant<int, N + decltype(u_c)::value>{});
+          });
+        }
+        if constexpr (LOAD && Q % 4 == 1 && Q / 4 < kL) dma(into, t_load, Q / 4);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    };
+    // Prologue: stage data 0 and 1 in flight, the first 16 elements split.
+#pragma unroll
+    for (int q = 0; q < kL; ++q) dma(st0, 0, q);
+#pragma unroll
+    for (int q = 0; q < kL; ++q) dma(st1, 1, q);
+    wait_vm_barrier<kL>();
+    static_for<kFr>([&](auto f_c) __attribute__((always_inline)) {
+      read_raw(st0, 0, decltype(f_c)::value);
+      static_for<kOps>([&](auto n_c) __attribute__((always_inline)) { split_op(S0{}, f_c, n_c); });
+    });
+    // Stage t: step 0 computes its first half and splits its second; then every
+    // wave has read the stage and, past the barrier, step 1 refills it with stage
+    // data t + 2 while it splits the first half of stage t + 1.  Past the last
+    // stage the loads and the split repeat the last stage's data, unused.
+    auto stage2 = [&](int t, auto s_c) __attribute__((always_inline)) {
+      constexpr int S = decltype(s_c)::value;
+      unsigned char* cur = stage_ptr(S);
+      step16(S0{}, cur, 1, F_{}, cur, 0);
+      wait_vm_barrier<0>();
+      step16(S1{}, stage_ptr(S ^ 1), 0, T_{}, cur, t + 2 < nst ? t + 2 : nst - 1);
+    };
+    for (int t = 0; t < nst; t += kStages) {
+      stage2(t, S0{});
+      stage2(t + 1, S1{});
+    }
+    wait_vm_barrier<0>();
+    // Infinities and NaN do not split (inf - inf), a value that rounds up to
+    // infinity does not either, and of values below 2^-109 the last plane falls
+    // under the smallest bf16: a tile in which one shows is formed again with fp32
+    // MFMAs.
+    constexpr uint32_t kLeast = 2u * (18u << 7) - 1u;  // 2^-109
+    float z = 0.f;
+#pragma unroll
+    for (int i = 0; i < kTM; ++i)
+#pragma unroll
+      for (int j = 0; j < kTN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) z += acc[i][j][v] * 0.f;
+    if (__syncthreads_or(!(z == 0.f) || (least & 0xffffu) < kLeast || (least >> 16) < kLeast)) {
+#pragma unroll
+      for (int i = 0; i < kTM; ++i)
+#pragma unroll
+        for (int j = 0; j < kTN; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+      run_stages();
+    }
+  } else {
+    run_stages();
   }
-  step(t, S0{}, T_{}, F_{});
-  step(t + 1, S1{}, F_{}, F_{});
 
   if constexpr (MODE == kGemm) {
     // ---- plain GEMM: the accumulators go straight to C ----

@@ -28,7 +28,7 @@ is ``[V, H]``; targets are ``[B, S]``.
 * fp32 hidden states and weights keep the reference's chunked shape on this
   library's kernels: per chunk of sequence positions the fp32 logits are one
   product on the same MFMA tile loop with fp32 operands (``mirl_gemm_f32_abt``,
-  four ``v_mfma_f32_32x32x2_f32`` per 16-byte fragment pair; the reference's
+  each fp32 product as six products of bf16 planes; the reference's
   ``torch.matmul`` output), and the row kernels of the logits path
   (``mirl_logprob_fwd`` / ``mirl_logprob_bwd``) form the logprobs and, in
   place, the logits gradient.  The backward moves the rows with a non-zero
@@ -36,7 +36,7 @@ is ``[V, H]``; targets are ``[B, S]``.
   block of one chunk of rows it recomputes their logits, forms G in place,
   and runs ``dH = G . W`` and ``dW += G^T . H`` in fp32 on the same tile loop
   (fp32 transposed copies of W, of the active hidden rows and of G).  An fp32
-  GEMM here is bound by the fp32 MFMA rate (1/16 of bf16's) at over a
+  GEMM here is bound by the MFMA rate (six bf16 products each) at over a
   thousand flops per byte of logits, so the per-chunk logits write and read
   that a fused epilogue would save cost under 1% of the step; skipping the
   rows with a zero upstream gradient saves most of the backward's products.
