@@ -473,6 +473,118 @@ __global__ __launch_bounds__(kFlatThreads) void logprob_bwd_flat_kernel(FlatBwd 
   bwd_flat_piece<E, kFlatThreads, kFlatVecs>(A, blockIdx.x);
 }
 
+// The flat schedule for rows that do not start on 16-byte boundaries (V not a
+// multiple of the vector width): the same 4 KB pieces over the flat array of
+// aligned vectors, of which one per row may hold the end of that row and the
+// start of the next.  V is at least a piece, so a piece meets at most two rows:
+// both rows' data are uniform (scalar) loads, each lane takes one of them, and
+// the lane whose vector straddles the boundary mixes them element by element.
+// Elements past the last whole vector are the next lane's.  Same arithmetic as
+// logprob_bwd_flat_kernel.  Measured on [3, 1021, 100003] bf16, 44% of the rows
+// active: 147 us, 6.0 TB/s; the two row-per-workgroup launches 198 us, 4.45 TB/s
+// ([4, 300, 5001], half active: 8.2 and 13.8 us).  Where V is a multiple of the
+// vector, logprob_bwd_flat_kernel's lookups per lane are cheaper (1.23 against
+// 1.32 ms on the [8, 2048, 151936] rows): no piece needs two rows' data there.
+template <class E>
+__global__ __launch_bounds__(kFlatThreads) void logprob_bwd_ragged_kernel(FlatBwd A, uint32_t rows,
+                                                                          double inv_v, double inv_rt) {
+  using raw = typename E::raw;
+  constexpr int NT = kFlatThreads, U = kFlatVecs, VEC = E::kVec;
+  const int64_t V = A.V, nelem = (int64_t)rows * V, nvec = nelem / VEC;
+  const vu4* xv = static_cast<const vu4*>(A.logits);
+  vu4* yv = static_cast<vu4*>(A.gin);
+  const int64_t v0 = (int64_t)blockIdx.x * (NT * U) - A.shift;
+  // the piece's first row, and where the next one starts.  Quotients by a product
+  // with the reciprocal, off by at most one: an integer division in front of every
+  // piece's loads cost a tenth of the kernel.
+  auto quotient = [](int64_t n, int64_t d, double inv) {
+    uint32_t q = (uint32_t)((double)n * inv);
+    const int64_t r = n - (int64_t)q * d;
+    return r < 0 ? q - 1 : r >= d ? q + 1 : q;
+  };
+  const uint32_t row0 = quotient(v0 > 0 ? v0 * VEC : 0, V, inv_v);
+  const int64_t bound = (int64_t)(row0 + 1) * V;
+  struct RowData {
+    float gv, M, LS;
+    int64_t target;  // flat element of the target, or -1
+  };
+  RowData d0{0.f, 0.f, 0.f, -1}, d1 = d0;
+  if (A.R > 0) {
+    // both rows' loads go out together, from clamped positions
+    float gv[2], M[2], LS[2];
+    int64_t t[2];
+    bool in[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const uint32_t row = row0 + k < rows ? row0 + k : rows - 1;
+      const uint32_t b = quotient(row, A.Rt, inv_rt);
+      const int64_t r0 = row - b * A.Rt, r = r0 < A.R ? r0 : A.R - 1;
+      in[k] = row0 + k < rows && r0 < A.R;
+      const int64_t srow = (int64_t)b * A.R + r;
+      gv[k] = A.g[(int64_t)b * A.gsb + r * A.gsr];
+      M[k] = A.stats[2 * srow];
+      LS[k] = A.stats[2 * srow + 1];
+      t[k] = A.target[(int64_t)b * A.tsb + r * A.tsr];
+    }
+    auto take = [&](int k) {
+      const bool hit = t[k] >= A.vs && t[k] < A.ve && t[k] - A.vs < V;
+      return RowData{in[k] ? gv[k] : 0.f, M[k], LS[k],
+                     hit ? (int64_t)(row0 + k) * V + (t[k] - A.vs) : -1};
+    };
+    d0 = take(0);
+    d1 = take(1);
+  }
+  auto grad = [&](float x, const RowData& d, int64_t e) {
+    const float p = fast_exp2(((x - d.M) - d.LS) * kLog2e);
+    return d.gv == 0.f ? 0.f : e == d.target ? (1.f - p) * d.gv : p * -d.gv;
+  };
+  vu4 q[U];
+  bool live[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t i = v0 + threadIdx.x + u * NT, e = i * VEC;
+    const bool in0 = e < bound, in1 = e + VEC > bound;
+    live[u] = i >= 0 && i < nvec && ((in0 && d0.gv != 0.f) || (in1 && d1.gv != 0.f));
+    if (live[u]) q[u] = __builtin_nontemporal_load(xv + i);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t i = v0 + threadIdx.x + u * NT, e = i * VEC;
+    if (i < 0 || i > nvec) continue;
+    if (i == nvec) {
+      // fewer elements than a vector are left; they end the last row
+      const raw* x = static_cast<const raw*>(A.logits);
+      raw* y = static_cast<raw*>(A.gin);
+      for (int64_t k = e; k < nelem; ++k) {
+        const RowData& d = k < bound ? d0 : d1;
+        y[k] = E::from_float(d.gv == 0.f ? 0.f : grad(E::load(x + k), d, k));
+      }
+      continue;
+    }
+    if (!live[u]) {
+      __builtin_nontemporal_store(vu4{0u, 0u, 0u, 0u}, yv + i);
+      continue;
+    }
+    float w[VEC], o[VEC];
+    E::unpack(q[u], w);
+    if (e < bound && e + VEC > bound) {
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) o[k] = grad(w[k], e + k < bound ? d0 : d1, e + k);
+    } else {
+      const bool first = e < bound;
+      const float gv = first ? d0.gv : d1.gv, M = first ? d0.M : d1.M, LS = first ? d0.LS : d1.LS;
+      const int64_t tj = (first ? d0.target : d1.target) - e;
+      const float ng = -gv;
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) o[k] = fast_exp2(((w[k] - M) - LS) * kLog2e) * ng;
+#pragma unroll
+      for (int k = 0; k < VEC; ++k)
+        if (k == tj) o[k] = (1.f - fast_exp2(((w[k] - M) - LS) * kLog2e)) * gv;
+    }
+    __builtin_nontemporal_store(E::pack(o), yv + i);
+  }
+}
+
 // The early-backward recheck's redo on the flat schedule.  Launches with no
 // flag set are the common case, and their cost is the number of (empty)
 // workgroups dispatched; the redo itself is fastest with one workgroup per
@@ -875,6 +987,24 @@ void dispatch_gather_fwd(int w, int64_t rows, hipStream_t st, const void* logits
   }
 }
 
+// The gradient is one contiguous [rows, V] array, the logits have its layout (or
+// are not read), and both start on 16-byte boundaries.
+bool flat_layout(int64_t rows, const void* logits, int64_t R, int64_t Rt, int64_t V, int64_t sb,
+                 int64_t sr, const void* gin, int64_t gisb, int64_t gisr) {
+  const uintptr_t ya = reinterpret_cast<uintptr_t>(gin), xa = reinterpret_cast<uintptr_t>(logits);
+  const bool contiguous = gisr == V && (rows == Rt || gisb == Rt * V);
+  const bool shared_layout = R == 0 || (sr == gisr && (rows == Rt || sb == gisb));
+  return contiguous && shared_layout && (ya & 15u) == 0 && (xa & 15u) == 0 && rows < (int64_t(1) << 31);
+}
+
+// Vectors by which the first piece starts ahead of the gradient, so that the pieces
+// start on 4 KB addresses.
+int flat_shift(const void* gin) {
+  constexpr int P = kFlatThreads * kFlatVecs;
+  const int to4k = (int)(((4096u - (reinterpret_cast<uintptr_t>(gin) & 4095u)) & 4095u) / 16u);
+  return (P - to4k) & (P - 1);
+}
+
 // The flat backward applies when gradient and logits share one contiguous,
 // 16-byte aligned [B, Rt, V] layout with whole vectors per row and the vector
 // count fits 32-bit indexing; fills the launch arguments and the piece count.
@@ -885,17 +1015,13 @@ bool flat_bwd_layout(int64_t rows, const void* logits, int64_t R, int64_t Rt, in
                      int64_t gsr, void* gin, int64_t gisb, int64_t gisr, FlatBwd* A,
                      int64_t* npieces) {
   constexpr int VEC = E::kVec;
-  const uintptr_t ya = reinterpret_cast<uintptr_t>(gin), xa = reinterpret_cast<uintptr_t>(logits);
-  const bool contiguous = gisr == V && (rows == Rt || gisb == Rt * V);
-  const bool shared_layout = R == 0 || (sr == gisr && (rows == Rt || sb == gisb));
   const int64_t nvr = V / VEC;
   const int64_t nvec = rows * nvr;
-  if (!(V % VEC == 0 && contiguous && shared_layout && (ya & 15u) == 0 && (xa & 15u) == 0 &&
-        nvec + 512 < (int64_t(1) << 32) && rows < (int64_t(1) << 31)))
+  if (!(V % VEC == 0 && flat_layout(rows, logits, R, Rt, V, sb, sr, gin, gisb, gisr) &&
+        nvec + 512 < (int64_t(1) << 32)))
     return false;
   constexpr int P = kFlatThreads * kFlatVecs;  // vectors per 4 KB piece
-  const int to4k = (int)(((4096u - (ya & 4095u)) & 4095u) / 16u);  // vectors before a 4 KB boundary
-  const int shift = (P - to4k) & (P - 1);
+  const int shift = flat_shift(gin);
   *npieces = (nvec + shift + P - 1) / P;
   *A = FlatBwd{logits, R, (uint32_t)Rt, (uint32_t)nvr, (uint32_t)nvec, shift, target, tsb, tsr,
                vs, ve, V, stats, g, gsb, gsr, gin, nullptr};
@@ -979,6 +1105,19 @@ void dispatch_bwd(int64_t rows, hipStream_t st, const void* logits, int64_t R, i
                          gsr, gin, gisb, gisr, &A, &npieces)) {
     hipLaunchKernelGGL((logprob_bwd_flat_kernel<E>), dim3((unsigned)npieces), dim3(kFlatThreads), 0,
                        st, A);
+    return;
+  }
+  // rows at other offsets of the same contiguous layout; below a piece's elements a
+  // piece would meet more than two rows
+  constexpr int P = kFlatThreads * kFlatVecs;
+  if (V >= P * E::kVec &&
+      flat_layout(rows, logits, R, Rt, V, sb, sr, gin, gisb, gisr) && rows * V / E::kVec + 512 < (int64_t(1) << 32)) {
+    const int shift = flat_shift(gin);
+    A = FlatBwd{logits, R, (uint32_t)Rt, 0, 0, shift, target, tsb, tsr,
+                vs, ve, V, stats, g, gsb, gsr, gin, nullptr};
+    npieces = (rows * V / E::kVec + 1 + shift + P - 1) / P;  // the leftover elements count as a vector
+    hipLaunchKernelGGL((logprob_bwd_ragged_kernel<E>), dim3((unsigned)npieces), dim3(kFlatThreads), 0, st,
+                       A, (uint32_t)rows, 1.0 / (double)V, 1.0 / (double)Rt);
     return;
   }
   hipLaunchKernelGGL((logprob_bwd_kernel<E, W, U, kZeroRows>), dim3((unsigned)rows), dim3(64 * W),
