@@ -1643,10 +1643,11 @@ __global__ __launch_bounds__(kPcThreads) void filter_bwd_piece_kernel(FilterBwdP
 
 // Per row with a rank-form cut and rcut > 0 (one wave each): the pieces'
 // tie counts scanned in order, and the listed ties of rank < rcut written as
-// zeros (a piece whose list overflowed is read again, its ties ranked by
-// ballot).  Measured on the top-p backward of bf16 [4, 4096, 151936] rows
-// (about 75 zeros per row): 0.17 ms, the cost of that many scattered 2-byte
-// writes into lines already written back.  A decoupled look-back in the piece
+// zeros (a piece whose list overflowed is read again whole, 128 bytes a lane, its
+// ties ranked by a wave scan; with 64 elements a step and a round trip each, the few
+// such pieces of a launch took most of it).  Measured on the top-p backward of bf16
+// [2, 2048, 151936] rows: 130 -> 30 us; [4, 4096, 151936]: 0.17 -> 0.05 ms.  Bound by the
+// latency of a row's dependent loads and of its scattered 2-byte stores.  A decoupled look-back in the piece
 // kernel (each piece adding up the counts its row's earlier pieces publish,
 // so that every tie is written once) measured 2.9 ms for the piece kernel
 // alone: pieces waiting on pieces of other XCDs hold their slots.
@@ -1655,6 +1656,8 @@ __global__ __launch_bounds__(256) void filter_bwd_piece_fixup_kernel(FilterBwdPa
                                                                      int64_t nrows) {
   using raw = typename E::raw;
   constexpr int VEC = E::kVec;
+  constexpr int kLV = kPcVectors / 64;  // vectors per lane of a piece read again
+  static_assert(kLV * VEC <= 64, "a lane's ties fit one mask");
   const int lane = threadIdx.x & 63;
   const int64_t srow = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (srow >= nrows) return;
@@ -1694,14 +1697,39 @@ __global__ __launch_bounds__(256) void filter_bwd_piece_fixup_kernel(FilterBwdPa
       const int l = __ffsll((unsigned long long)ov) - 1;
       const int pv = c0 + l;
       uint32_t rk = (uint32_t)__shfl((int)start, l, 64);
-      const int64_t j0 = piece_j0(Gm, pv, VEC);
-      const int64_t j1 = pv == Gm.ppr - 1 ? P.V : (int64_t)Gm.head + (int64_t)(pv + 1) * kPcVectors * VEC;
-      for (int64_t jj = j0; jj < j1 && rk < rcut; jj += 64) {
-        const int64_t j = jj + lane;
+      // single elements j < j1 before the first vector or after the last
+      auto loose = [&](int64_t j, int64_t j1) {
         const bool tie = j < j1 && W.yval(E::load(x + j)) == W.vc;
         const uint64_t bal = __ballot(tie);
         if (tie && rk + (uint32_t)__popcll(bal & below) < rcut) y[j] = zr;
         rk += (uint32_t)__popcll(bal);
+      };
+      if (pv == 0) loose(lane, Gm.head);
+      // the body: each lane reads its kLV vectors in one go and ranks its ties
+      // after those of the lanes before it
+      const int i0 = pv * kPcVectors + lane * kLV;
+      const vu4* xv = reinterpret_cast<const vu4*>(x + Gm.head);
+      vu4 q[kLV];
+#pragma unroll
+      for (int v = 0; v < kLV; ++v) q[v] = i0 + v < Gm.nvec ? xv[i0 + v] : vu4{0u, 0u, 0u, 0u};
+      uint64_t ties = 0ull;
+#pragma unroll
+      for (int v = 0; v < kLV; ++v) {
+        float w[VEC];
+        E::unpack(q[v], w);
+#pragma unroll
+        for (int k = 0; k < VEC; ++k)
+          ties |= (uint64_t)(i0 + v < Gm.nvec && W.yval(w[k]) == W.vc) << (v * VEC + k);
+      }
+      const uint32_t nt = (uint32_t)__popcll(ties);
+      const uint32_t it = wave_scan_dpp(nt);
+      raw* yb = y + Gm.head + (int64_t)i0 * VEC;
+      for (uint32_t at = rk + it - nt; ties != 0ull && at < rcut; ties &= ties - 1ull, ++at)
+        yb[__ffsll((unsigned long long)ties) - 1] = zr;
+      rk += (uint32_t)__shfl((int)it, 63, 64);
+      if (pv == Gm.ppr - 1) {
+        const int64_t tail0 = (int64_t)Gm.head + (int64_t)Gm.nvec * VEC;
+        loose(tail0 + lane, P.V);
       }
     }
     seen += (uint32_t)__shfl((int)inc, 63, 64);
