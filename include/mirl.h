@@ -526,6 +526,21 @@ int mirl_gemm_f32_abt(const float* A, int64_t lda, const float* B, int64_t ldb, 
                       int accumulate, const int64_t* count, int64_t count_off, int count_axis,
                       void* stream);
 
+/* The rows of the hidden-state backward whose upstream gradient is not zero, moved to
+ * the front in order (grad_out [B, S] fp32 by strides, row r = (s, b) = (r / bsz, r % bsz)):
+ * perm [T] the permutation (the other rows follow in any order), *count the number of
+ * such rows (a device int64), grad_rows [T] / target_out [T] / stats_out [T, 2] the rows'
+ * upstream gradients, targets and forward statistics in that order, hidden_out [T, Hd]
+ * contiguous the hidden rows m < *count (rows past it are not written).
+ * Replaces: the masking of rows in ChunkedDistributedHiddenStatesToLogprobs.backward
+ * (nemo_rl/distributed/model_utils.py:2647-2745), which forms them as zeros. */
+int mirl_lce_active_rows(const float* grad_out, int64_t g_stride_b, int64_t g_stride_s, int64_t T,
+                         int64_t bsz, const int64_t* target, int64_t t_stride_b,
+                         int64_t t_stride_s, const float* row_stats, const void* hidden,
+                         int dtype, int64_t Hd, int64_t ldh, int64_t* perm, int64_t* count,
+                         int64_t* target_out, float* stats_out, float* grad_rows,
+                         void* hidden_out, void* stream);
+
 /* out[r(m), n] = out_dtype(sum_s part[s, m, n]) summed in s order (part [k_splits][M][ld]
  * fp32, out row stride ldo, out_dtype MIRL_DTYPE_BF16, MIRL_DTYPE_F16 or
  * MIRL_DTYPE_F32): the splits of mirl_gemm_bf16_abt / mirl_gemm_f32_abt.  r(m) = out_rows[m]

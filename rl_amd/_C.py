@@ -235,6 +235,10 @@ SIGNATURES = {
     "mirl_gemm_f32_abt": (
         _I, [_P, _I64, _P, _I64, _I64, _I64, _I64, _I64, _P, _I64, _I, _P, _I64, _I, _P]
     ),
+    "mirl_lce_active_rows": (
+        _I,
+        [_P, _I64, _I64, _I64, _I64, _P, _I64, _I64, _P, _P, _I, _I64, _I64, _P, _P, _P, _P, _P, _P, _P],
+    ),
     "mirl_transpose_f32": (_I, [_P, _I64, _I64, _I64, _P, _I64, _I64, _P, _I64, _P]),
     "mirl_top_k_top_p_mask": (
         _I,
@@ -1310,6 +1314,34 @@ def gemm_f32_abt(a: torch.Tensor, b: torch.Tensor, k: int, out: torch.Tensor, k_
         int(count_axis), _stream(dev),
     )
     _check(st, "mirl_gemm_f32_abt")
+
+
+def lce_active_rows(grad_out: torch.Tensor, target: torch.Tensor, stats: torch.Tensor,
+                    hidden2d: torch.Tensor) -> tuple[torch.Tensor, ...]:
+    """(perm [T], count [1], hidden rows [T, H], targets [1, T], stats [T, 2], gradients [1, T]) of
+    the rows r = s * B + b with a non-zero grad_out[b, s] moved to the front; hidden rows past
+    the count are left unwritten."""
+    dev = _require_gpu(grad_out, target, stats, hidden2d)
+    B, S = target.shape
+    T, H = hidden2d.shape
+    _require(T == S * B and tuple(grad_out.shape) == (B, S), "a gradient and a target per hidden row")
+    _require(grad_out.dtype == torch.float32 and target.dtype == torch.int64, "fp32 gradients, int64 targets")
+    _require(stats.dtype == torch.float32 and stats.is_contiguous() and stats.numel() == 2 * T,
+             "contiguous fp32 row statistics")
+    _require(hidden2d.stride(-1) == 1, "unit stride on the last dim")
+    ints = torch.empty(2 * T + 1, dtype=torch.int64, device=dev)
+    perm, tgt, count = ints[:T], ints[T : 2 * T], ints[2 * T :]
+    floats = torch.empty(3 * T, dtype=torch.float32, device=dev)
+    st_a, g_a = floats[: 2 * T], floats[2 * T :]
+    h_a = torch.empty((T, H), dtype=hidden2d.dtype, device=dev)
+    st = _launch(
+        "mirl_lce_active_rows", dev, grad_out.data_ptr(), grad_out.stride(0), grad_out.stride(1), T, B,
+        target.data_ptr(), target.stride(0), target.stride(1), stats.data_ptr(), hidden2d.data_ptr(),
+        _dtype_code(hidden2d), H, hidden2d.stride(0), perm.data_ptr(), count.data_ptr(), tgt.data_ptr(),
+        st_a.data_ptr(), g_a.data_ptr(), h_a.data_ptr(), _stream(dev),
+    )
+    _check(st, "mirl_lce_active_rows")
+    return perm, count, h_a, tgt.view(1, T), st_a.view(T, 2), g_a.view(1, T)
 
 
 def transpose_f32(src: torch.Tensor, rows: int, dst: torch.Tensor, count: Optional[torch.Tensor] = None,

@@ -1018,6 +1018,79 @@ __global__ __launch_bounds__(256) void sum_splits_kernel(const float* __restrict
   }
 }
 
+// The rows r = (s, b) = (r / bsz, r % bsz) whose upstream gradient is not zero, in
+// order, then the others from the end backwards: perm, the rows' gradients and the
+// count of the first kind.  One workgroup, 8 x 1024 rows a step (their loads in
+// flight together, a ballot and a sum over 16 waves per 1024).  With the gather below
+// it takes the place of a stable sort, a sum and six gathers of the library: step of
+// 137 rows x [1355, 4096] fp16 356 -> 248 us (host-bound), of 115 rows x [11749, 4096]
+// bf16 441 -> 337; nothing to see at 16384 rows.
+constexpr int kActThreads = 1024;
+__global__ __launch_bounds__(kActThreads) void lce_active_rows_kernel(
+    const float* __restrict__ g, int64_t gsb, int64_t gss, uint32_t T, uint32_t bsz,
+    int64_t* __restrict__ perm, float* __restrict__ g_a, int64_t* __restrict__ count) {
+  constexpr int NW = kActThreads / kWave, U = 8;
+  __shared__ uint32_t wsum[2][NW];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  uint32_t base = 0;  // active rows before this step
+  for (uint32_t r0 = 0; r0 < T; r0 += U * kActThreads) {
+    float v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t r = r0 + u * kActThreads + tid;
+      const uint32_t s = r / bsz, b = r - s * bsz;
+      v[u] = r < T ? g[(int64_t)b * gsb + (int64_t)s * gss] : 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t r = r0 + u * kActThreads + tid;
+      const bool act = r < T && v[u] != 0.f;
+      const uint64_t bal = __ballot(act);
+      // the two buffers alternate, so one barrier a round separates a round's
+      // writes from the reads of the round before last
+      if (lane == 0) wsum[u & 1][wave] = (uint32_t)__popcll(bal);
+      __syncthreads();
+      uint32_t before = base + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const uint32_t n = wsum[u & 1][w];
+        before += w < wave ? n : 0u;
+        base += n;
+      }
+      if (r < T) {
+        const uint32_t at = act ? before : T - 1 - (r - before);
+        perm[at] = r;
+        g_a[at] = v[u];
+      }
+    }
+  }
+  if (tid == 0) *count = base;
+}
+
+// Row m of the permuted targets and statistics and, for m < *count, of the permuted
+// hidden states (row_units units of UNIT per row; rows past the count stay as they
+// are: every kernel stops at the count).  One workgroup per row.
+template <class UNIT>
+__global__ __launch_bounds__(256) void lce_gather_rows_kernel(
+    const int64_t* __restrict__ perm, const int64_t* __restrict__ count, uint32_t bsz,
+    const int64_t* __restrict__ target, int64_t tsb, int64_t tss, const float* __restrict__ stats,
+    const UNIT* __restrict__ hidden, int64_t row_units, int64_t ld_units, int64_t* __restrict__ tgt_a,
+    float* __restrict__ st_a, UNIT* __restrict__ h_a) {
+  const int64_t m = blockIdx.x;
+  const uint32_t r = (uint32_t)perm[m];
+  const bool live = m < *count;
+  if (threadIdx.x == 0) {
+    const uint32_t s = r / bsz, b = r - s * bsz;
+    tgt_a[m] = target[(int64_t)b * tsb + (int64_t)s * tss];
+    st_a[2 * m] = stats[2 * (int64_t)r];
+    st_a[2 * m + 1] = stats[2 * (int64_t)r + 1];
+  }
+  if (!live) return;
+  const UNIT* src = hidden + (int64_t)r * ld_units;
+  UNIT* dst = h_a + m * row_units;
+  for (int64_t k = threadIdx.x; k < row_units; k += 256) dst[k] = src[k];
+}
+
 // Per row: combine the column-tile partials into the row's max and log-sum-exp,
 // then logprob = (x_t - max) - logsum (0 for targets outside the slice).
 // One wave per row.
@@ -1380,6 +1453,49 @@ extern "C" int mirl_gemm_f32_abt(const float* A, int64_t lda, const float* B, in
   hipLaunchKernelGGL((lce_tile_kernel<kGemm, F32>), dim3((unsigned)grid), dim3(kThreads), 0,
                      static_cast<hipStream_t>(stream), P);
   return check_launch("mirl_gemm_f32_abt");
+}
+
+extern "C" int mirl_lce_active_rows(const float* grad_out, int64_t g_stride_b, int64_t g_stride_s,
+                                    int64_t T, int64_t bsz, const int64_t* target,
+                                    int64_t t_stride_b, int64_t t_stride_s, const float* row_stats,
+                                    const void* hidden, int dtype, int64_t Hd, int64_t ldh,
+                                    int64_t* perm, int64_t* count, int64_t* target_out,
+                                    float* stats_out, float* grad_rows, void* hidden_out,
+                                    void* stream) {
+  clear_error();
+  MIRL_REQUIRE(lce_dtype_ok(dtype) || dtype == MIRL_DTYPE_F32,
+               "hidden states must be bf16, fp16 or fp32 (dtype code %d)", dtype);
+  MIRL_REQUIRE(T >= 0 && Hd > 0 && bsz > 0 && ldh >= Hd, "invalid shape T=%lld H=%lld B=%lld", (long long)T,
+               (long long)Hd, (long long)bsz);
+  MIRL_REQUIRE(T % bsz == 0, "row count %lld is not a multiple of the batch size %lld", (long long)T,
+               (long long)bsz);
+  MIRL_REQUIRE(T < (int64_t(1) << 31) - 8 * kActThreads, "too many rows (%lld)", (long long)T);
+  MIRL_REQUIRE(count != nullptr, "null pointer argument");
+  MIRL_REQUIRE(T == 0 || (grad_out && target && row_stats && hidden && perm && target_out && stats_out &&
+                          grad_rows && hidden_out),
+               "null pointer argument");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  hipLaunchKernelGGL(lce_active_rows_kernel, dim3(1), dim3(kActThreads), 0, st, grad_out, g_stride_b,
+                     g_stride_s, (uint32_t)T, (uint32_t)bsz, perm, grad_rows, count);
+  if (T > 0) {
+    const int64_t esz = dtype == MIRL_DTYPE_F32 ? 4 : 2;
+    const uintptr_t both = reinterpret_cast<uintptr_t>(hidden) | reinterpret_cast<uintptr_t>(hidden_out);
+    auto launch = [&](auto unit) {
+      using UNIT = decltype(unit);
+      constexpr int64_t n = sizeof(UNIT);
+      hipLaunchKernelGGL(lce_gather_rows_kernel<UNIT>, dim3((unsigned)T), dim3(256), 0, st, perm, count,
+                         (uint32_t)bsz, target, t_stride_b, t_stride_s, row_stats,
+                         static_cast<const UNIT*>(hidden), Hd * esz / n, ldh * esz / n, target_out,
+                         stats_out, static_cast<UNIT*>(hidden_out));
+    };
+    if ((both & 15u) == 0 && Hd * esz % 16 == 0 && ldh * esz % 16 == 0)
+      launch(vu4{});
+    else if (esz == 4)
+      launch(uint32_t{});
+    else
+      launch(uint16_t{});
+  }
+  return check_launch("mirl_lce_active_rows");
 }
 
 extern "C" int mirl_transpose_f32(const float* src, int64_t R, int64_t C, int64_t lds, float* dst,

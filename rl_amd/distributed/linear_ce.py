@@ -143,14 +143,7 @@ class ChunkedDistributedHiddenStatesToLogprobs(torch.autograd.Function):
         # zero.  The rows are permuted so that the active ones come first (in row
         # order) and their count stays on the device: every kernel below reads it
         # and skips what lies past it, so the host never waits for the count.
-        g_rows = grad_output.t().reshape(T)  # row r = (s, b) is position s of sample b
-        nz = g_rows != 0
-        perm = torch.argsort(torch.logical_not(nz).to(torch.uint8), stable=True)
-        count = nz.sum(dtype=torch.int64).view(1)
-        h_a = torch.index_select(h2, 0, perm)
-        tgt_a = target.t().reshape(T).index_select(0, perm).view(1, T)
-        st_a = stats.index_select(0, perm)
-        g_a = g_rows.index_select(0, perm).view(1, T)
+        perm, count, h_a, tgt_a, st_a, g_a = _C.lce_active_rows(grad_output, target, stats, h2)
         # Blocks of up to 4 chunks of rows (whole 256-row tiles): the bf16 G
         # buffer stays below one reference chunk's fp32 logits, softmax and
         # one-hot temporaries.  Blocks past the count return at once.
@@ -342,14 +335,7 @@ def _f32_backward(ctx, grad_output):
         grad_output = grad_output.float()
     need_h, need_w = ctx.needs_input_grad[0], ctx.needs_input_grad[2]
     h2 = hidden.view(T, H)
-    g_rows = grad_output.t().reshape(T)
-    nz = g_rows != 0
-    perm = torch.argsort(torch.logical_not(nz).to(torch.uint8), stable=True)
-    count = nz.sum(dtype=torch.int64).view(1)
-    h_a = torch.index_select(h2, 0, perm)
-    tgt_a = target.t().reshape(T).index_select(0, perm).view(1, T)
-    st_a = stats.index_select(0, perm)
-    g_a = g_rows.index_select(0, perm).view(1, T)
+    perm, count, h_a, tgt_a, st_a, g_a = _C.lce_active_rows(grad_output, target, stats, h2)
     hk_a, wk = _f32_operand(h_a), _f32_operand(weight)
     K = hk_a.shape[1]
     rows = T if ctx.chunk_size is None else min(T, _round_up(ctx.chunk_size * B, 256))
@@ -457,14 +443,17 @@ def _dh_splits(n: int, H: int, K: int, count_known: bool = True) -> int:
 
 
 _transpose_streams: dict = {}
+# Weights up to this many elements are transposed on the current stream: the transpose takes
+# at most 30 us there, what the side stream's events cost the host.
+_INLINE_TRANSPOSE = 1 << 25
 
 
 def _weight_transposed(weight: torch.Tensor, Vp: int):
     """W^T [H, Vp] bf16 (columns past V zero; an fp16 weight rounded), formed from the weight's current contents
     in every backward (one read and one write of W, about 0.5 ms at [151936, 4096]), and the event
-    that marks it written.
+    that marks it written (None where it was formed on the current stream).
 
-    The transpose runs on a side stream (default priority) behind everything already
+    A large weight's transpose runs on a side stream (default priority) behind everything already
     enqueued on the current stream, so it overlaps the gradient kernel, which is bound by
     the MFMA units; the caller waits for the event on the current stream before the first
     product that reads W^T.  The buffer is allocated on the current stream, which frees
@@ -476,6 +465,9 @@ def _weight_transposed(weight: torch.Tensor, Vp: int):
     V, H = weight.shape
     dev = weight.device
     wT = torch.empty((H, Vp), dtype=torch.bfloat16, device=dev)
+    if V * H <= _INLINE_TRANSPOSE:
+        _C.transpose_bf16(weight, V, wT)
+        return wT, None
     side = _transpose_streams.get(dev)
     if side is None:
         side = torch.cuda.Stream(dev)

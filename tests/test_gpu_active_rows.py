@@ -1,0 +1,37 @@
+"""The rows of the hidden-state backward with a non-zero upstream gradient, moved to the front,
+against torch on the CPU (GPU)."""
+
+import pytest
+import torch
+
+from rl_amd import _C
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+
+
+@pytest.mark.parametrize("S,B,H,pad", [(1, 1, 8, 0), (63, 1, 5, 0), (1023, 1, 16, 0), (512, 2, 24, 8), (205, 5, 7, 1),
+                                       (8192, 1, 8, 0), (2731, 3, 4, 0)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("share", [0.0, 0.3, 1.0])
+def test_active_rows(S, B, H, pad, dtype, share):
+    g = torch.Generator().manual_seed(S + B)
+    up = torch.randn(B, S + 1, generator=g) * (torch.rand(B, S + 1, generator=g) < share)
+    up = up[:, 1:]  # strided
+    if share > 0:
+        up[0, 0], up[-1, -1] = float("nan"), -0.0
+    target = torch.randint(-5, 1000, (B, S), generator=g)
+    T = S * B
+    stats = torch.randn(T, 2, generator=g)
+    wide = torch.randn(T, H + pad, generator=g).to(dtype)
+    hidden = wide.to(DEV)[:, :H]
+    perm, count, h, tgt, st, ga = (x.cpu() for x in _C.lce_active_rows(up.to(DEV), target.to(DEV), stats.to(DEV),
+                                                                       hidden))
+    rows = up.t().reshape(T)
+    active = (rows != 0).nonzero()[:, 0]
+    n = int(count)
+    assert n == active.numel()
+    assert torch.equal(perm[:n], active) and torch.equal(perm.sort().values, torch.arange(T))
+    assert torch.equal(h[:n], wide[:, :H][active])
+    assert torch.equal(tgt[0], target.t().reshape(T)[perm]) and torch.equal(st, stats[perm])
+    torch.testing.assert_close(ga[0], rows[perm], rtol=0, atol=0, equal_nan=True)
