@@ -14,7 +14,8 @@ is ``[V, H]``; targets are ``[B, S]``.
 * backward: the rows with a non-zero upstream gradient are moved to the front
   (the others have a zero logits gradient: zero dH rows, nothing added to dW)
   and counted on the device, where the kernels read the count (no host
-  synchronisation); per block of up to ``4 * chunk_size * B`` rows a kernel recomputes the logits
+  synchronisation); per block of ``4 * chunk_size * B`` rows (more where those leave CUs
+  idle, see ``_block_rows``) a kernel recomputes the logits
   tiles and writes ``G = (onehot - softmax) * g`` in bf16 and its transpose, and
   ``dH = G . W`` and ``dW += G^T . H`` run on the same MFMA tile loop
   (``mirl_gemm_bf16_abt``) against bf16 transposed copies of W (formed in every
@@ -26,14 +27,14 @@ is ``[V, H]``; targets are ``[B, S]``.
   tail, which together make up most of ``dH``; the transposes round fp16 W and
   H to bf16 for those two products.
 * fp32 hidden states and weights keep the reference's chunked shape on this
-  library's kernels: per chunk of sequence positions the fp32 logits are one
+  library's kernels: per block of at least a chunk's rows the fp32 logits are one
   product on the same MFMA tile loop with fp32 operands (``mirl_gemm_f32_abt``,
   each fp32 product as six products of bf16 planes; the reference's
   ``torch.matmul`` output), and the row kernels of the logits path
   (``mirl_logprob_fwd`` / ``mirl_logprob_bwd``) form the logprobs and, in
   place, the logits gradient.  The backward moves the rows with a non-zero
   upstream gradient to the front and counts them on the device, as above; per
-  block of one chunk of rows it recomputes their logits, forms G in place,
+  block of at least one chunk of rows it recomputes their logits, forms G in place,
   and runs ``dH = G . W`` and ``dW += G^T . H`` in fp32 on the same tile loop
   (fp32 transposed copies of W, of the active hidden rows and of G).  An fp32
   GEMM here is bound by the MFMA rate (six bf16 products each) at over a
@@ -147,7 +148,7 @@ class ChunkedDistributedHiddenStatesToLogprobs(torch.autograd.Function):
         # Blocks of up to 4 chunks of rows (whole 256-row tiles): the bf16 G
         # buffer stays below one reference chunk's fp32 logits, softmax and
         # one-hot temporaries.  Blocks past the count return at once.
-        rows = T if ctx.chunk_size is None else min(T, _round_up(_BLOCK_CHUNKS * ctx.chunk_size * B, 256))
+        rows = _block_rows(T, ctx.chunk_size, _BLOCK_CHUNKS * B, V)
         n_blocks = -(-T // rows)
         Vp = _round_up(V, _K_ALIGN)
         # G [rows, Vp] (columns past V zero: dH's padded reduction length)
@@ -286,8 +287,8 @@ def _f32_operand(x: torch.Tensor) -> torch.Tensor:
 
 
 def _f32_forward(ctx, hidden, target, weight, vs, ve, chunk_size, inference_only):
-    """fp32: per chunk of positions, logits = hidden[c] . weight^T (fp32 tile loop, rows in
-    (position, sample) order), then the logprob row kernel over them (reference
+    """fp32: per block of at least a chunk's rows, logits = hidden . weight^T (fp32 tile loop,
+    rows in (position, sample) order), then the logprob row kernel over them (reference
     model_utils.py:2608-2630).  The row statistics are saved per row r = s * B + b."""
     S, B, H = hidden.shape
     V = weight.shape[0]
@@ -299,11 +300,9 @@ def _f32_forward(ctx, hidden, target, weight, vs, ve, chunk_size, inference_only
     tgt_rows = target.t().reshape(1, T)  # row r = (s, b): position s of sample b
     out_rows = torch.empty((1, T), dtype=torch.float32, device=dev)
     stats = None if inference_only else torch.empty((T, 2), dtype=torch.float32, device=dev)
-    chunks = _chunks(S, chunk_size)
-    logits = torch.empty((max((c1 - c0) * B for c0, c1 in chunks), V), dtype=torch.float32, device=dev) \
-        if chunks else None
-    for c0, c1 in chunks:
-        r0, r1 = c0 * B, c1 * B
+    rows = _block_rows(T, chunk_size, B, V)
+    logits = torch.empty((rows, V), dtype=torch.float32, device=dev)
+    for r0, r1 in _chunks(T, rows):
         lc = logits[: r1 - r0]
         _C.gemm_f32_abt(h2[r0:r1], w2, K, lc)
         st_c = None if stats is None else stats[r0:r1].view(1, r1 - r0, 2)
@@ -338,7 +337,7 @@ def _f32_backward(ctx, grad_output):
     perm, count, h_a, tgt_a, st_a, g_a = _C.lce_active_rows(grad_output, target, stats, h2)
     hk_a, wk = _f32_operand(h_a), _f32_operand(weight)
     K = hk_a.shape[1]
-    rows = T if ctx.chunk_size is None else min(T, _round_up(ctx.chunk_size * B, 256))
+    rows = _block_rows(T, ctx.chunk_size, B, V)
     Vp = _round_up(V, _F32_K_ALIGN)
     L = torch.empty((rows, Vp), dtype=torch.float32, device=dev)  # logits, then G
     if Vp > V:
@@ -407,6 +406,19 @@ def _round_up(n: int, m: int) -> int:
     return (n + m - 1) // m * m
 
 
+def _block_rows(T: int, chunk_size: Optional[int], rows_per_position: int, V: int) -> int:
+    """Rows handled at a time: all of them without a chunk size, else those of a chunk
+    (``rows_per_position`` rows a position) in whole 256-row tiles, and at least as many as
+    give every CU two 256 x 256 tiles of the [rows, V] logits.  Fewer leave CUs idle and
+    tiles partly empty (64-row chunks of [512, 1024] x [32000, 1024] fp32: 2.2 ms of kernels;
+    the whole step takes 0.62 ms in one block); the scratch this adds is at most 512 such tiles (134 MB in fp32)
+    and one 256-row strip of the logits."""
+    if chunk_size is None:
+        return T
+    least = 256 * -(-512 // -(-V // 256))
+    return min(T, max(_round_up(chunk_size * rows_per_position, 256), least))
+
+
 def _padded_width(rows: int) -> int:
     """Row length of the transposed operands of dW: whole 256-row tiles plus one
     128-byte line, so that the rows a tile reads together do not all start at the
@@ -421,16 +433,26 @@ def _dh_splits(n: int, H: int, K: int, count_known: bool = True) -> int:
     tie (measured on [5871, 151936] x [151936, 4096]: 1 split 7.62 ms, 2 6.09,
     3 6.81, 4 6.23).  The kernel cuts K into ranges of round_up(ceil(K / s), 128);
     only counts for which that gives exactly s ranges, each of at least 1024, qualify.
+    With fewer than 32 tiles, eight ranges each do not fill the CUs once: as many as do
+    ([276, 151936] x [151936, 224], two tiles: 8 splits 0.4 ms; with 119 the whole step goes
+    from 767 to 468 us).
     With count_known False, n is an upper bound (the active rows are counted on the
     device) and at least two splits are taken where they qualify: fewer active rows
     leave the single-split tiles short of the CUs, and a second split costs one more
     fp32 partial of n x H."""
     tiles = ((n + 255) // 256) * ((H + 255) // 256)
+    def qualifies(s: int) -> bool:
+        kb = _round_up(-(-K // s), 128)
+        return kb >= 1024 and -(-K // kb) == s
+
+    if tiles < 32:
+        for s in range(min(256 // max(tiles, 1), K // 1024), 8, -1):
+            if qualifies(s):
+                return s
     best, best_eff = 1, tiles / (256 * -(-tiles // 256))
     qualifying = []
     for s in range(2, 9):
-        kb = _round_up(-(-K // s), 128)
-        if kb < 1024 or -(-K // kb) != s:
+        if not qualifies(s):
             continue
         qualifying.append(s)
         t = tiles * s
