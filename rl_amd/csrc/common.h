@@ -175,6 +175,14 @@ struct RowSpan {
   }
 };
 
+// n / d for 0 <= n < 2^53 and a quotient below 2^32, by a product with inv = 1.0 / d
+// (off by at most one before the correction).
+__device__ __forceinline__ uint32_t quotient(int64_t n, int64_t d, double inv) {
+  const uint32_t q = (uint32_t)((double)n * inv);
+  const int64_t r = n - (int64_t)q * d;
+  return r < 0 ? q - 1 : r >= d ? q + 1 : q;
+}
+
 // fp32 value rounded to the element type and widened back.
 template <class E>
 __device__ __forceinline__ float round_trip(float f) {

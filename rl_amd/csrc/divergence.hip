@@ -355,6 +355,88 @@ __global__ __launch_bounds__(kDivFlatThreads) void divergence_bwd_flat_kernel(
   }
 }
 
+// The flat schedule for rows that do not start on 16-byte boundaries (V not a multiple
+// of the vector width, at least a piece long, so that a piece meets at most two rows).
+// Both rows' data are uniform loads and each lane takes one of them; the lane whose
+// vector holds the end of one row and the start of the next mixes them element by
+// element, and the elements past the last whole vector are the next lane's.  Same
+// arithmetic as divergence_bwd_flat_kernel.  Bound by memory: reverse KL of bf16
+// [2, 1200, 100003], 44% of the rows active: 161 us, 5.6 TB/s; a workgroup per row
+// 237 us, 3.8 TB/s.
+template <class E, int KIND>
+__global__ __launch_bounds__(kDivFlatThreads) void divergence_bwd_ragged_kernel(
+    const typename E::raw* __restrict__ xs, const typename E::raw* __restrict__ xt, int64_t V,
+    uint32_t rows, int shift, const float* __restrict__ Lrow, const float* __restrict__ stats,
+    const float* __restrict__ g, uint32_t R, int64_t gsb, int64_t gsr, typename E::raw* gin,
+    double inv_v, double inv_r) {
+  constexpr bool kTeacher = DivTraits<KIND>::kTeacher;
+  constexpr int VEC = E::kVec;
+  constexpr int NT = kDivFlatThreads, U = 2;
+  const vu4* xv = reinterpret_cast<const vu4*>(xs);
+  const vu4* tv = reinterpret_cast<const vu4*>(xt);
+  vu4* yv = reinterpret_cast<vu4*>(gin);
+  const int64_t nelem = (int64_t)rows * V, nvec = nelem / VEC;
+  const int64_t v0 = (int64_t)blockIdx.x * (NT * U) - shift;
+  const uint32_t row0 = quotient(v0 > 0 ? v0 * VEC : 0, V, inv_v);
+  const int64_t bound = (int64_t)(row0 + 1) * V;  // where the piece's second row starts
+  struct RowData {
+    float g, M, LZ, Mt, LZt, L;
+  } d[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const uint32_t row = row0 + k < rows ? row0 + k : rows - 1;
+    const uint32_t b = quotient(row, R, inv_r), r = row - b * R;
+    const float* o = stats + 4 * (int64_t)row;
+    d[k] = RowData{g[(int64_t)b * gsb + (int64_t)r * gsr], o[0], o[1], o[2], o[3], Lrow[row]};
+  }
+  const RowData d0 = d[0], d1 = d[1];
+  auto grad = [&](float x, float t, const RowData& e) {
+    return e.g == 0.f ? 0.f : div_grad<KIND>(x, t, e.M, e.LZ, e.Mt, e.LZt, e.L, e.g);
+  };
+  vu4 q[U], qt[U];
+  bool live[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t i = v0 + threadIdx.x + u * NT, e = i * VEC;
+    live[u] = i >= 0 && i < nvec && ((e < bound && d0.g != 0.f) || (e + VEC > bound && d1.g != 0.f));
+    if (live[u]) {
+      q[u] = __builtin_nontemporal_load(xv + i);
+      if constexpr (kTeacher) qt[u] = __builtin_nontemporal_load(tv + i);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t i = v0 + threadIdx.x + u * NT, e = i * VEC;
+    if (i < 0 || i > nvec) continue;
+    if (i == nvec) {
+      // fewer elements than a vector are left; they end the last row
+      for (int64_t k = e; k < nelem; ++k) {
+        const RowData& c = k < bound ? d0 : d1;
+        gin[k] = E::from_float(
+            c.g == 0.f ? 0.f : grad(E::load(xs + k), kTeacher ? E::load(xt + k) : 0.f, c));
+      }
+      continue;
+    }
+    if (!live[u]) {
+      __builtin_nontemporal_store(vu4{0u, 0u, 0u, 0u}, yv + i);
+      continue;
+    }
+    float w[VEC], wt[VEC], o[VEC];
+    E::unpack(q[u], w);
+    if constexpr (kTeacher) E::unpack(qt[u], wt);
+    if (e < bound && e + VEC > bound) {
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) o[k] = grad(w[k], kTeacher ? wt[k] : 0.f, e + k < bound ? d0 : d1);
+    } else {
+      const RowData c = e < bound ? d0 : d1;
+#pragma unroll
+      for (int k = 0; k < VEC; ++k)
+        o[k] = div_grad<KIND>(w[k], kTeacher ? wt[k] : 0.f, c.M, c.LZ, c.Mt, c.LZt, c.L, c.g);
+    }
+    __builtin_nontemporal_store(E::pack(o), yv + i);
+  }
+}
+
 // Row-per-workgroup backward for any strides (vector body when the student,
 // teacher and gradient rows are co-aligned, element-wise otherwise).
 template <class E, int KIND>
@@ -456,18 +538,26 @@ void dispatch_bwd(int64_t rows, hipStream_t st, const void* xs, const void* xt, 
   // every [B, R, V] array contiguous with the same layout
   const bool contig = gisr == V && gisb == R * V && ssr == V && ssb == R * V &&
                       (!kTeacher || (tsr == V && tsb == R * V));
-  const int64_t nvr = V / VEC;
-  const int64_t nvec = rows * nvr;
-  if (V % VEC == 0 && contig && (ya & 15u) == 0 && (xa & 15u) == 0 &&
+  constexpr int P = kDivFlatThreads * 2;  // vectors per 4 KB piece
+  const int64_t nvec = rows * V / VEC;
+  // below a piece's elements a ragged piece would meet more than two rows
+  if (contig && (V % VEC == 0 || V >= P * VEC) && (ya & 15u) == 0 && (xa & 15u) == 0 &&
       (!kTeacher || (ta & 15u) == 0) && nvec + 512 < (int64_t(1) << 32)) {
     const int to4k = (int)(((4096u - (ya & 4095u)) & 4095u) / 16u);
-    constexpr int P = kDivFlatThreads * 2;  // vectors per 4 KB piece
     const int shift = (P - to4k) & (P - 1);
-    const int64_t grid = (nvec + shift + P - 1) / P;
-    hipLaunchKernelGGL((divergence_bwd_flat_kernel<E, KIND>), dim3((unsigned)grid),
-                       dim3(kDivFlatThreads), 0, st, static_cast<const raw*>(xs),
-                       static_cast<const raw*>(xt), (uint32_t)nvr, (uint32_t)nvec, shift, L, stats,
-                       g, R, gsb, gsr, static_cast<raw*>(gin));
+    const auto *x = static_cast<const raw*>(xs), *t = static_cast<const raw*>(xt);
+    if (V % VEC == 0) {
+      const int64_t grid = (nvec + shift + P - 1) / P;
+      hipLaunchKernelGGL((divergence_bwd_flat_kernel<E, KIND>), dim3((unsigned)grid),
+                         dim3(kDivFlatThreads), 0, st, x, t, (uint32_t)(V / VEC), (uint32_t)nvec,
+                         shift, L, stats, g, R, gsb, gsr, static_cast<raw*>(gin));
+    } else {
+      const int64_t grid = (nvec + 1 + shift + P - 1) / P;  // the leftover elements count as a vector
+      hipLaunchKernelGGL((divergence_bwd_ragged_kernel<E, KIND>), dim3((unsigned)grid),
+                         dim3(kDivFlatThreads), 0, st, x, t, V, (uint32_t)rows, shift, L, stats, g,
+                         (uint32_t)R, gsb, gsr, static_cast<raw*>(gin), 1.0 / (double)V,
+                         1.0 / (double)R);
+    }
     return;
   }
   hipLaunchKernelGGL((divergence_bwd_row_kernel<E, KIND>), dim3((unsigned)rows), dim3(256), 0, st,

@@ -497,11 +497,6 @@ __global__ __launch_bounds__(kFlatThreads) void logprob_bwd_ragged_kernel(FlatBw
   // the piece's first row, and where the next one starts.  Quotients by a product
   // with the reciprocal, off by at most one: an integer division in front of every
   // piece's loads cost a tenth of the kernel.
-  auto quotient = [](int64_t n, int64_t d, double inv) {
-    uint32_t q = (uint32_t)((double)n * inv);
-    const int64_t r = n - (int64_t)q * d;
-    return r < 0 ? q - 1 : r >= d ? q + 1 : q;
-  };
   const uint32_t row0 = quotient(v0 > 0 ? v0 * VEC : 0, V, inv_v);
   const int64_t bound = (int64_t)(row0 + 1) * V;
   struct RowData {
