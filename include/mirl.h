@@ -339,8 +339,8 @@ int mirl_filtered_logprob_fwd(const void* logits, int dtype, int64_t B, int64_t 
  * and the kept entries stored; otherwise the rows are rewritten whole, each
  * row written once); any value gives the same gradient.
  * workspace (or NULL): mirl_filtered_logprob_bwd_workspace_bytes(dtype, B, R, V)
- * bytes.  With it, rows without kept lists whose logits and gradient rows all
- * start at the same offset from a 16-byte boundary are written in 8 KB pieces
+ * bytes.  With it, rows without kept lists whose logits start at the same
+ * offset from a 16-byte boundary as their gradient are written in 8 KB pieces
  * in address order; the ties of a cut in rank form are counted and listed
  * there per piece and settled by a per-row pass.  Without it (or for other
  * layouts) a workgroup walks each row.  Either way the gradient is the same.

@@ -1431,7 +1431,10 @@ __global__ __launch_bounds__(kRowThreads, 6) void filter_bwd_row_kernel(FilterBw
 // together).  Measured on the top-k 2000 backward of bf16 [4, 4096, 151936]
 // rows (9.48 GB): 1.49 ms on 8 KB pieces, 1.83 ms on 4 KB pieces (a piece's
 // dependent loads amortized over half the bytes), 1.65 ms on 16 KB pieces;
-// 2.10 ms for the row walk.
+// 2.10 ms for the row walk.  Rows that each start at another offset from a 16-byte
+// boundary (V not a multiple of a vector), top-p backward of bf16 [4, 600, 100003]:
+// 144 us and 8 us of fix-up, 192 us for the row walk; 151 us with pieces that start
+// on the rows' vectors instead of on 128-byte lines.
 //
 // A cut in index form (j kept among the elements equal to v_cut from i_cut
 // on) is applied per element.  In rank form (kept among those ties from rank
@@ -1443,21 +1446,39 @@ __global__ __launch_bounds__(kRowThreads, 6) void filter_bwd_row_kernel(FilterBw
 constexpr int kPcThreads = 256;
 constexpr int kPcVecs = 2;                          // 16-byte vectors per thread
 constexpr int kPcVectors = kPcThreads * kPcVecs;    // per piece
+constexpr int kPcLine = 8;                          // vectors of a 128-byte line
 constexpr int kPieceTieCap = MIRL_FILTER_PIECE_TIE_CAP;
 static_assert(kPieceTieCap % 2 == 0, "a piece's list is read as 32-bit words");
 
 struct PieceGeom {
-  int ppr;            // pieces per row
-  int nvec;           // 16-byte vectors per row (the same in every row)
-  int head;           // elements before the first vector
+  int ppr;            // pieces per row (the most that a row of V elements can have)
   uint32_t* tie_cnt;  // [B * R * ppr]: the piece's tie count (rank-form rows with rcut > 0)
   uint16_t* tie_pos;  // [B * R * ppr][kPieceTieCap]: tie offsets from the piece's first element
 };
 
-// first element of piece pc (piece 0 starts at the row's element 0)
-__device__ __forceinline__ int piece_j0(const PieceGeom& Gm, int pc, int vec) {
-  return pc == 0 ? 0 : Gm.head + pc * kPcVectors * vec;
-}
+// A row's elements before its first 16-byte vector, its vectors, and the first element
+// after them.  They differ from row to row where V is not a multiple of a vector.  Pieces
+// start on 128-byte lines: the first one `skew` vectors before the row's first, so that
+// no line but a row's first and last is written by two workgroups.  The last piece may be
+// without any vector and still write the elements after them.
+template <class E>
+struct PieceRow {
+  int head, nvec, tail0, skew;
+  __device__ __forceinline__ PieceRow(const typename E::raw* y, int64_t V) {
+    const RowSpan<E> s(y, V);
+    head = (int)s.head;
+    nvec = (int)s.nvec;
+    tail0 = (int)s.tail0;
+    skew = (int)(reinterpret_cast<uintptr_t>(y + head) >> 4) & (kPcLine - 1);
+  }
+  // the vector at which piece pc starts
+  __device__ __forceinline__ int first(int pc) const { return pc * kPcVectors - skew; }
+  // first element of piece pc (piece 0 starts at the row's element 0)
+  __device__ __forceinline__ int j0(int pc) const {
+    return pc == 0 ? 0 : min(head + first(pc) * E::kVec, tail0);
+  }
+  __device__ __forceinline__ bool holds(int i) const { return (uint32_t)i < (uint32_t)nvec; }
+};
 
 template <class E, int CONV>
 __global__ __launch_bounds__(kPcThreads) void filter_bwd_piece_kernel(FilterBwdParams P, PieceGeom Gm) {
@@ -1482,27 +1503,28 @@ __global__ __launch_bounds__(kPcThreads) void filter_bwd_piece_kernel(FilterBwdP
     t = P.target[(int64_t)b * P.tsb + (int64_t)r * P.tsr];
   }
   raw* y = static_cast<raw*>(P.gin) + (int64_t)b * P.gisb + (int64_t)r * P.gisr;
-  vu4* yv = reinterpret_cast<vu4*>(y + Gm.head);
-  const int i0 = pc * kPcVectors + tid;  // this thread's first vector
-  const int tail0 = Gm.head + Gm.nvec * VEC;
-  const bool hv = pc == 0 && tid < Gm.head;                         // a head element
+  const PieceRow<E> Rw(y, P.V);
+  vu4* yv = reinterpret_cast<vu4*>(y + Rw.head);
+  const int i0 = Rw.first(pc) + tid;  // this thread's first vector
+  const int tail0 = Rw.tail0;
+  const bool hv = pc == 0 && tid < Rw.head;                         // a head element
   const bool tv = pc == Gm.ppr - 1 && tail0 + tid < (int)P.V;       // a tail element
   const raw zr = E::from_float(0.f);
   if (gv == 0.f) {
     // rows past R and rows with a zero upstream gradient: zeros, the logits unread
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (i0 + u * NT < Gm.nvec) __builtin_nontemporal_store(vu4{0u, 0u, 0u, 0u}, yv + i0 + u * NT);
+      if (Rw.holds(i0 + u * NT)) __builtin_nontemporal_store(vu4{0u, 0u, 0u, 0u}, yv + i0 + u * NT);
     if (hv) y[tid] = zr;
     if (tv) y[tail0 + tid] = zr;
     return;
   }
   const raw* x = static_cast<const raw*>(P.logits) + (int64_t)b * P.sb + (int64_t)r * P.sr;
-  const vu4* xv = reinterpret_cast<const vu4*>(x + Gm.head);
+  const vu4* xv = reinterpret_cast<const vu4*>(x + Rw.head);
   vu4 q[U];
 #pragma unroll
   for (int u = 0; u < U; ++u)
-    q[u] = i0 + u * NT < Gm.nvec ? __builtin_nontemporal_load(xv + i0 + u * NT) : vu4{0u, 0u, 0u, 0u};
+    q[u] = Rw.holds(i0 + u * NT) ? __builtin_nontemporal_load(xv + i0 + u * NT) : vu4{0u, 0u, 0u, 0u};
   const float xh = hv ? E::load(x + tid) : 0.f;
   const float xt = tv ? E::load(x + tail0 + tid) : 0.f;
   const WalkMath<E, CONV> W(P, ri, gv, t);
@@ -1519,7 +1541,7 @@ __global__ __launch_bounds__(kPcThreads) void filter_bwd_piece_kernel(FilterBwdP
       w[u][k] = W.yval(w[u][k]);
       a = a || w[u][k] == vc;
     }
-    anyt[u] = a && i0 + u * NT < Gm.nvec;
+    anyt[u] = a && Rw.holds(i0 + u * NT);
   }
   auto tie_bits = [&](int u) {
     uint32_t m = 0u;
@@ -1545,7 +1567,7 @@ __global__ __launch_bounds__(kPcThreads) void filter_bwd_piece_kernel(FilterBwdP
     const int icut = W.icut;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int jb = Gm.head + (i0 + u * NT) * VEC;
+      const int jb = Rw.head + (i0 + u * NT) * VEC;
       if (jb + VEC <= icut) thr[u] = vnext;
       const bool cutvec = jb < icut && jb + VEC > icut && anyt[u];
       if (__ballot(cutvec) != 0ull && cutvec) drop[u] = tie_bits(u) & ((1u << (icut - jb)) - 1u);
@@ -1589,7 +1611,7 @@ __global__ __launch_bounds__(kPcThreads) void filter_bwd_piece_kernel(FilterBwdP
     }
     // the count and the list (offsets in index order, up to kPieceTieCap)
     const uint64_t below = (1ull << lane) - 1ull;
-    const int j0 = piece_j0(Gm, pc, VEC);
+    const int j0 = Rw.j0(pc);
     const int64_t slot = (int64_t)srow * Gm.ppr + pc;
     uint16_t* lst = Gm.tie_pos + slot * kPieceTieCap;
     if (th) {
@@ -1598,7 +1620,7 @@ __global__ __launch_bounds__(kPcThreads) void filter_bwd_piece_kernel(FilterBwdP
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int jb = Gm.head + (i0 + u * NT) * VEC;
+      const int jb = Rw.head + (i0 + u * NT) * VEC;
       uint32_t a = before[u];
       for (uint32_t m = tb[u]; m != 0u; m &= m - 1u, ++a) {
         const int k = __ffs(m) - 1;
@@ -1615,7 +1637,7 @@ __global__ __launch_bounds__(kPcThreads) void filter_bwd_piece_kernel(FilterBwdP
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int i = i0 + u * NT;
-    const int jb = Gm.head + i * VEC;
+    const int jb = Rw.head + i * VEC;
     float o[VEC];
 #pragma unroll
     for (int k = 0; k < VEC; ++k) o[k] = w[u][k] >= thr[u] ? W.prob(w[u][k]) * ngv : 0.f;
@@ -1635,7 +1657,7 @@ __global__ __launch_bounds__(kPcThreads) void filter_bwd_piece_kernel(FilterBwdP
         }
     }
     const vu4 out = W.pack_vec(o);
-    if (i < Gm.nvec) __builtin_nontemporal_store(out, yv + i);
+    if (Rw.holds(i)) __builtin_nontemporal_store(out, yv + i);
   }
   if (hv) y[tid] = W.grad_at(yh, tid, yh > vc || keepH);
   if (tv) y[tail0 + tid] = W.grad_at(ytl, tail0 + tid, ytl > vc || keepTl);
@@ -1669,6 +1691,7 @@ __global__ __launch_bounds__(256) void filter_bwd_piece_fixup_kernel(FilterBwdPa
   const uint32_t rcut = (uint32_t)(-1 - ri.i_cut);
   raw* y = static_cast<raw*>(P.gin) + b * P.gisb + r * P.gisr;
   const raw* x = static_cast<const raw*>(P.logits) + b * P.sb + r * P.sr;
+  const PieceRow<E> Rw(y, P.V);
   const raw zr = E::from_float(0.f);
   const WalkMath<E, CONV> W(P, ri, gv, -1);
   const uint32_t* cnt = Gm.tie_cnt + srow * Gm.ppr;
@@ -1683,7 +1706,7 @@ __global__ __launch_bounds__(256) void filter_bwd_piece_fixup_kernel(FilterBwdPa
     const bool need = n > 0u && start < rcut;
     if (need && n <= (uint32_t)kPieceTieCap) {
       // the piece's list read whole (independent loads), then the zeros stored
-      const int j0 = piece_j0(Gm, pc, VEC);
+      const int j0 = Rw.j0(pc);
       const uint32_t m = min(n, rcut - start);
       const uint32_t* pw = reinterpret_cast<const uint32_t*>(pos + pc * kPieceTieCap);
       uint32_t wv[kPieceTieCap / 2];
@@ -1704,14 +1727,14 @@ __global__ __launch_bounds__(256) void filter_bwd_piece_fixup_kernel(FilterBwdPa
         if (tie && rk + (uint32_t)__popcll(bal & below) < rcut) y[j] = zr;
         rk += (uint32_t)__popcll(bal);
       };
-      if (pv == 0) loose(lane, Gm.head);
+      if (pv == 0) loose(lane, Rw.head);
       // the body: each lane reads its kLV vectors in one go and ranks its ties
       // after those of the lanes before it
-      const int i0 = pv * kPcVectors + lane * kLV;
-      const vu4* xv = reinterpret_cast<const vu4*>(x + Gm.head);
+      const int i0 = Rw.first(pv) + lane * kLV;
+      const vu4* xv = reinterpret_cast<const vu4*>(x + Rw.head);
       vu4 q[kLV];
 #pragma unroll
-      for (int v = 0; v < kLV; ++v) q[v] = i0 + v < Gm.nvec ? xv[i0 + v] : vu4{0u, 0u, 0u, 0u};
+      for (int v = 0; v < kLV; ++v) q[v] = Rw.holds(i0 + v) ? xv[i0 + v] : vu4{0u, 0u, 0u, 0u};
       uint64_t ties = 0ull;
 #pragma unroll
       for (int v = 0; v < kLV; ++v) {
@@ -1719,18 +1742,15 @@ __global__ __launch_bounds__(256) void filter_bwd_piece_fixup_kernel(FilterBwdPa
         E::unpack(q[v], w);
 #pragma unroll
         for (int k = 0; k < VEC; ++k)
-          ties |= (uint64_t)(i0 + v < Gm.nvec && W.yval(w[k]) == W.vc) << (v * VEC + k);
+          ties |= (uint64_t)(Rw.holds(i0 + v) && W.yval(w[k]) == W.vc) << (v * VEC + k);
       }
       const uint32_t nt = (uint32_t)__popcll(ties);
       const uint32_t it = wave_scan_dpp(nt);
-      raw* yb = y + Gm.head + (int64_t)i0 * VEC;
+      raw* yb = y + Rw.head + (int64_t)i0 * VEC;
       for (uint32_t at = rk + it - nt; ties != 0ull && at < rcut; ties &= ties - 1ull, ++at)
         yb[__ffsll((unsigned long long)ties) - 1] = zr;
       rk += (uint32_t)__shfl((int)it, 63, 64);
-      if (pv == Gm.ppr - 1) {
-        const int64_t tail0 = (int64_t)Gm.head + (int64_t)Gm.nvec * VEC;
-        loose(tail0 + lane, P.V);
-      }
+      if (pv == Gm.ppr - 1) loose(Rw.tail0 + lane, P.V);
     }
     seen += (uint32_t)__shfl((int)inc, 63, 64);
   }
@@ -1883,34 +1903,29 @@ int launch_topk_export(const FilterParams& P, int64_t rows, hipStream_t st) {
   return check_launch("topk_export_general_kernel");
 }
 
-// Pieces per row bound (16-byte vectors of V elements, 4 KB pieces), for the workspace size.
+// The most pieces that a row of V elements can have, whatever line its first vector starts in.
 int64_t piece_ppr_bound(int64_t V, int64_t esz) {
   const int64_t nv = V * esz / 16;
-  return nv > 0 ? (nv + kPcVectors - 1) / kPcVectors : 1;
+  return nv > 0 ? (nv + kPcLine - 1 + kPcVectors - 1) / kPcVectors : 1;
 }
 
-// The piece schedule's geometry when the layout allows it (logits and gradient
-// co-aligned, every row at the same 16-byte offset, rows whole in 32-bit
+// The piece schedule's geometry when the layout allows it (each row of the logits and
+// its gradient at the same offset from a 16-byte boundary, rows whole in 32-bit
 // indexing), else ppr = 0.
 template <class E>
 PieceGeom piece_geom(const FilterBwdParams& P, int64_t B, int64_t rows, void* ws) {
   PieceGeom Gm{};
   constexpr int64_t esz = sizeof(typename E::raw);
   const uintptr_t ax = reinterpret_cast<uintptr_t>(P.logits), ay = reinterpret_cast<uintptr_t>(P.gin);
-  auto row_step_ok = [&](int64_t stride, int64_t extent) { return extent <= 1 || (stride * esz) % 16 == 0; };
-  if (ws == nullptr || ax % esz != 0 || ay % esz != 0 || ax % 16 != ay % 16) return Gm;
-  if (!row_step_ok(P.sb, B) || !row_step_ok(P.sr, P.R) || !row_step_ok(P.gisb, B) || !row_step_ok(P.gisr, P.Rt))
-    return Gm;
-  int64_t head = (int64_t)(((16u - (ay & 15u)) & 15u) / esz);
-  if (head > P.V) head = P.V;
-  const int64_t nvec = (P.V - head) / E::kVec;
-  const int64_t ppr = nvec > 0 ? (nvec + kPcVectors - 1) / kPcVectors : 1;
+  auto steps_ok = [&](int64_t s, int64_t gs, int64_t extent) { return extent <= 1 || ((s - gs) * esz) % 16 == 0; };
+  if (ws == nullptr || ax % esz != 0 || ay % esz != 0) return Gm;
+  // without rows to read (R = 0) the logits' place does not matter
+  if (P.R > 0 && (ax % 16 != ay % 16 || !steps_ok(P.sb, P.gisb, B) || !steps_ok(P.sr, P.gisr, P.R))) return Gm;
+  const int64_t ppr = piece_ppr_bound(P.V, esz);
   if (rows * ppr * kPcThreads >= (int64_t(1) << 32)) return Gm;
   // workspace: the tie counts, then the tie lists
-  const int64_t slots = B * P.R * piece_ppr_bound(P.V, esz);
+  const int64_t slots = B * P.R * ppr;
   Gm.ppr = (int)ppr;
-  Gm.nvec = (int)nvec;
-  Gm.head = (int)head;
   Gm.tie_cnt = static_cast<uint32_t*>(ws);
   Gm.tie_pos = reinterpret_cast<uint16_t*>(Gm.tie_cnt + slots);
   return Gm;

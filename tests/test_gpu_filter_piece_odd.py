@@ -1,0 +1,51 @@
+"""The filtered backward's 8 KB pieces over rows that each start at another offset from a
+16-byte boundary (V not a multiple of a vector), against the row-per-workgroup walk (GPU).
+
+The sizes put the last piece's end around a piece's 512 vectors: rows of one launch with a
+last piece that holds vectors and with one that holds only the elements after them.
+"""
+
+import pytest
+import torch
+
+from rl_amd import _C
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+
+
+@pytest.mark.parametrize("dtype,V", [(torch.bfloat16, 5), (torch.bfloat16, 13), (torch.bfloat16, 4095),
+                                     (torch.bfloat16, 4099), (torch.bfloat16, 4105), (torch.bfloat16, 4107),
+                                     (torch.bfloat16, 38931), (torch.float16, 4107), (torch.float32, 2047),
+                                     (torch.float32, 2053), (torch.float32, 20002)])
+@pytest.mark.parametrize("tied", [1, 8, 400])  # elements per distinct value: listed ties, and lists that overflow
+@pytest.mark.parametrize("T", [1.0, 0.7])
+def test_pieces_equal_walk(dtype, V, tied, T):
+    B, S = 2, 17
+    g = torch.Generator().manual_seed(V + tied)
+    x = torch.randn(B, S, V, generator=g)
+    if tied > 1:
+        step = 8.0 * tied / V
+        x = (x / step).round() * step
+    x = x.to(dtype).to(DEV)
+    tgt = torch.randint(0, V, (B, S - 1), generator=g)
+    tgt[0, :2] = torch.tensor([0, V - 1])
+    up = torch.randn(B, S - 1, generator=g)
+    up[:, 3:6] = 0.0
+    tgt, up = tgt.to(DEV), up.to(DEV)
+    decision = torch.float32 if dtype != torch.float32 else None
+    for p in (0.9, 0.4):
+        info, kidx, kp = _C.filtered_fwd(x, tgt, T, 0, p, None, decision)
+        out = []
+        for pieces in (True, False):
+            store = torch.full((B * S * V + 64,), 7.0, dtype=dtype, device=DEV)
+            grad = store[:B * S * V].view(B, S, V)
+            _C.filtered_bwd(x, tgt, T, info, kidx, kp, up, grad, top_k=0, pieces=pieces)
+            assert torch.all(store[B * S * V:] == 7.0)
+            out.append(grad)
+        assert torch.equal(out[0], out[1])
+        assert not out[0][:, -1].any() and not out[0][:, 3:6].any()
+        # rows of another stride at the same offsets
+        wide = torch.full((B, S, V + 16), 7.0, dtype=dtype, device=DEV)[..., :V]
+        _C.filtered_bwd(x, tgt, T, info, kidx, kp, up, wide, top_k=0)
+        assert torch.equal(wide, out[0])
