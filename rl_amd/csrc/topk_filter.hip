@@ -1465,10 +1465,12 @@ template <class E>
 struct PieceRow {
   int head, nvec, tail0, skew;
   __device__ __forceinline__ PieceRow(const typename E::raw* y, int64_t V) {
-    const RowSpan<E> s(y, V);
-    head = (int)s.head;
-    nvec = (int)s.nvec;
-    tail0 = (int)s.tail0;
+    // (RowSpan in 32 bits, V < 2^31: a piece is short enough for scalar work to show)
+    const uint32_t v = (uint32_t)V, vec = E::kVec;
+    const uint32_t h = min((0u - (uint32_t)reinterpret_cast<uintptr_t>(y) & 15u) / (16u / vec), v);
+    head = (int)h;
+    nvec = (int)((v - h) / vec);
+    tail0 = head + nvec * (int)vec;
     skew = (int)(reinterpret_cast<uintptr_t>(y + head) >> 4) & (kPcLine - 1);
   }
   // the vector at which piece pc starts
@@ -1921,7 +1923,14 @@ PieceGeom piece_geom(const FilterBwdParams& P, int64_t B, int64_t rows, void* ws
   if (ws == nullptr || ax % esz != 0 || ay % esz != 0) return Gm;
   // without rows to read (R = 0) the logits' place does not matter
   if (P.R > 0 && (ax % 16 != ay % 16 || !steps_ok(P.sb, P.gisb, B) || !steps_ok(P.sr, P.gisr, P.R))) return Gm;
-  const int64_t ppr = piece_ppr_bound(P.V, esz);
+  int64_t ppr = piece_ppr_bound(P.V, esz);
+  if ((B <= 1 || P.gisb * esz % 128 == 0) && (P.Rt <= 1 || P.gisr * esz % 128 == 0)) {
+    // every row starts at the same place of a line: no piece more than they need
+    // (131072 elements in 32 pieces: an empty 33rd cost the kernel 6%)
+    const int64_t head = std::min<int64_t>((16 - ay % 16) % 16 / esz, P.V), nvec = (P.V - head) / E::kVec;
+    const int64_t skew = (int64_t)(ay / 16 + (ay % 16 != 0)) % kPcLine;
+    ppr = std::max<int64_t>(1, (nvec + skew + kPcVectors - 1) / kPcVectors);
+  }
   if (rows * ppr * kPcThreads >= (int64_t(1) << 32)) return Gm;
   // workspace: the tie counts, then the tie lists
   const int64_t slots = B * P.R * ppr;
