@@ -199,6 +199,23 @@ __device__ __forceinline__ T wave_scan_dpp(T v, Op op = Op()) {
   return v;
 }
 
+// The same over each row of 16 lanes alone.
+template <class T, class Op = OpAdd>
+__device__ __forceinline__ T row16_scan(T v, Op op = Op()) {
+  v = op(v, dpp_move<0x111>(v));
+  v = op(v, dpp_move<0x112>(v));
+  v = op(v, dpp_move<0x114>(v));
+  return op(v, dpp_move<0x118>(v));
+}
+// Lane `l`'s value, as a scalar (l the same in every lane).
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, int l) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
+}
+__device__ __forceinline__ double lane_value(double v, int l) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, ((uint64_t)lane_value((uint32_t)(u >> 32), l) << 32) | lane_value((uint32_t)u, l));
+}
+
 // Forward over 16-bit logits by the histogram kernel (topk_hist.hip): every
 // row when all_rows != 0, else only the rows whose info.flags bit 0 is set.
 int launch_hist_rows(const FilterParams& P, int dtype, int64_t rows, int all_rows,

@@ -171,18 +171,16 @@ __device__ uint32_t block_max_u(uint32_t v, uint32_t* red) {
 // invocation, so no barrier is needed before it is written.
 template <class T, int NW>
 __device__ __forceinline__ T block_excl_scan1(T v, T* red, T* total) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  static_assert(NW <= 16, "the waves' sums are scanned in a row of 16 lanes");
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const T inc = wave_scan_dpp(v);
   if (lane == 63) red[wv] = inc;
   __syncthreads();
-  T base = T(0), tot = T(0);
-#pragma unroll
-  for (int w = 0; w < NW; ++w) {
-    const T s = red[w];
-    base += (w < wv) ? s : T(0);
-    tot += s;
-  }
-  *total = tot;
+  const T wave = lane < NW ? red[lane] : T(0);  // lane w takes wave w's sum
+  const T incl = row16_scan(wave);
+  *total = lane_value(incl, NW - 1);
+  // the sums of the waves before this one, by the scan's own association
+  const T base = wv > 0 ? lane_value(incl, wv - 1) : T(0);
   return base + inc - v;
 }
 // Workgroup-wide sums of N values with one barrier (`red`: N * NW entries,
@@ -197,12 +195,7 @@ __device__ __forceinline__ void block_sum1(T (&v)[N], T* red) {
   }
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < N; ++i) {
-    T s = T(0);
-#pragma unroll
-    for (int w = 0; w < NW; ++w) s += red[i * NW + w];
-    v[i] = s;
-  }
+  for (int i = 0; i < N; ++i) v[i] = lane_value(row16_scan(lane < NW ? red[i * NW + lane] : T(0)), NW - 1);
 }
 
 // Relative distance within which the fp32 running sum S is kept from the
@@ -920,6 +913,13 @@ __global__ __launch_bounds__(kHT) void filter_hist_kernel(FilterParams P, int64_
 //    (two values at a time), an address and an increment.  A value outside
 //    the window (|x| >= 512, +-inf, NaN) lands in word 0x4400 and flags the
 //    row for filter_hist_kernel.
+// What a row costs besides its count (cycles of its workgroup, fp16 [8, 1500, 38930],
+// 11500 distinct values, top-p): clearing 2200, listing 12300, the entries' values 5800,
+// normaliser 2300, cut 6400, group 6300, against 11500 for the count; with every thread
+// passing over all CMAX slots of its share in each phase, the group's exponentials formed
+// again and the waves' sums added up by every thread it was 59800 in place of 47600
+// altogether (kernel 1199 -> 987 us; the window form on bf16 [2, 2400, 32000] 38500 ->
+// 36600).  Bound by instruction issue in these phases, by the LDS counters in the count.
 struct CompactFull {
   static constexpr int NT = 1024;
   static constexpr uint32_t kBase = 0;      // first key of the table
@@ -1168,23 +1168,27 @@ __global__ __launch_bounds__(G::NT, 2048 / G::NT) void filter_compact_kernel(Fil
     const uint32_t kneg = wneg != 0u ? 0x7fffu - (L0 + (uint32_t)kWPT - wneg) : 0u;
     kloc = kpos != 0u ? kpos : kneg;  // key 0 (the largest NaN) orders below every other
   } else {
-    uint32_t kpos = 0;
-#pragma unroll 8
+    // per word: the count and the occupied halves as above, and the last occupied
+    // word and what it holds
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    uint32_t occ = 0, wl = 0, wlast = 0;
+#pragma unroll
     for (int w = 0; w < kWPT; ++w) {
-      const uint32_t lo = wd[w] & 0xffffu, hi = wd[w] >> 16;
-      ct += lo + hi;
-      nzp += (lo != 0u ? 1u : 0u) + (hi != 0u ? 1u : 0u);
-      if (lo != 0u) kpos = key0 + 2u * (uint32_t)w;
-      if (hi != 0u) kpos = key0 + 2u * (uint32_t)w + 1u;
+      ct = __builtin_amdgcn_sad_u16(wd[w], 0u, ct);
+      occ += __builtin_bit_cast(
+          uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, wd[w]), (u16x2)(uint16_t)1));
+      wl = wd[w] != 0u ? (uint32_t)w : wl;
+      wlast = wd[w] != 0u ? wd[w] : wlast;
     }
-    kloc = kpos;
+    nzp = (occ & 0xffffu) + (occ >> 16);
+    kloc = wlast != 0u ? key0 + 2u * wl + (wlast > 0xffffu ? 1u : 0u) : 0u;
   }
   // one barrier for the entry offsets, the numbers of entries, the total
   // count and the largest occupied key
   uint32_t N, Nn, tot, kmx;
   uint32_t off_p, off_n;
   {
-    const int lane = tid & 63, wv = tid >> 6;
+    const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t ip = wave_scan_dpp(nzp);
     const uint32_t in_ = wave_scan_dpp(nzn);
     const uint32_t ict = wave_scan_dpp(ct);
@@ -1196,21 +1200,17 @@ __global__ __launch_bounds__(G::NT, 2048 / G::NT) void filter_compact_kernel(Fil
       sh.red_u[3 * NW + wv] = ikm;
     }
     __syncthreads();
-    uint32_t bp = 0u, bn = 0u, Np = 0u;
-    Nn = 0u;
-    tot = 0u;
-    kmx = 0u;
+    // lane w takes wave w's values: a scan over a row of 16 lanes places the waves
+    static_assert(NW <= 16, "one row of 16 lanes");
+    uint32_t v[4];
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const uint32_t a = sh.red_u[w], an = sh.red_u[NW + w];
-      bp += (w < wv) ? a : 0u;
-      bn += (w < wv) ? an : 0u;
-      Np += a;
-      Nn += an;
-      tot += sh.red_u[2 * NW + w];
-      kmx = max(kmx, sh.red_u[3 * NW + w]);
-    }
-    N = Np + Nn;
+    for (int q = 0; q < 4; ++q) v[q] = lane < NW ? sh.red_u[q * NW + lane] : 0u;
+    const uint32_t sp_ = row16_scan(v[0]), sn = row16_scan(v[1]);
+    Nn = lane_value(sn, NW - 1);
+    N = lane_value(sp_, NW - 1) + Nn;
+    tot = lane_value(row16_scan(v[2]), NW - 1);
+    kmx = lane_value(row16_scan(v[3], OpMaxU()), NW - 1);
+    const uint32_t bp = lane_value(sp_ - v[0], wv), bn = lane_value(sn - v[1], wv);
     off_p = Nn + bp + ip - nzp;  // the positive (or key-layout) entries, ascending
     off_n = Nn - (bn + in_);     // the negative entries of later threads come first
   }
@@ -1250,7 +1250,7 @@ __global__ __launch_bounds__(G::NT, 2048 / G::NT) void filter_compact_kernel(Fil
         j += lo != 0u ? 1u : 0u;
       }
     }
-  } else {
+  } else if (nzp != 0u) {
     uint32_t j = off_p;
 #pragma unroll
     for (int w = 0; w < kWPT; ++w) {
@@ -1269,6 +1269,10 @@ __global__ __launch_bounds__(G::NT, 2048 / G::NT) void filter_compact_kernel(Fil
   constexpr int CMAX = (kEntCap + NT - 1) / NT;
   const uint32_t C = (N + NT - 1) / NT;  // the same for every thread
   const uint32_t j0 = min(N, (uint32_t)tid * C), j1 = min(N, j0 + C);
+  // The loops over a share stop, kGroup entries at a time, at the shares' common length
+  // C (a scalar): half of CMAX and less where the row has few distinct values.
+  constexpr int kGroup = 3;
+  auto past = [&](int i) { return i % kGroup == 0 && (uint32_t)i >= C; };
   uint32_t rn[CMAX];  // counts, 0 past the share
   float re[CMAX];     // exp(y - m)
 #pragma unroll
@@ -1303,6 +1307,15 @@ __global__ __launch_bounds__(G::NT, 2048 / G::NT) void filter_compact_kernel(Fil
   // first entry in [lo, hi] whose y >= v (hi + 1 if none); last entry whose y <= v (lo - 1 if none)
   auto first_ge = [&](uint32_t lo, uint32_t hi, float v) {
     uint32_t a = lo, c = hi + 1u;
+    // (the groups are a few entries: steps that double, from hi down)
+    for (uint32_t d = 1u; a < c; d <<= 1) {
+      const uint32_t t = c - lo > d ? c - d : lo;
+      if (!(yat(t) >= v)) {
+        a = t + 1u;
+        break;
+      }
+      c = t;
+    }
     while (a < c) {
       const uint32_t mid = (a + c) >> 1;
       if (yat(mid) >= v) c = mid; else a = mid + 1u;
@@ -1311,6 +1324,14 @@ __global__ __launch_bounds__(G::NT, 2048 / G::NT) void filter_compact_kernel(Fil
   };
   auto last_le = [&](uint32_t lo, uint32_t hi, float v) {
     uint32_t a = lo, c = hi + 1u;
+    for (uint32_t d = 1u; a < c; d <<= 1) {
+      const uint32_t t = c - a > d ? a + d - 1u : hi;
+      if (!(yat(t) <= v)) {
+        c = t;
+        break;
+      }
+      a = t + 1u;
+    }
     while (a < c) {
       const uint32_t mid = (a + c) >> 1;
       if (yat(mid) <= v) a = mid + 1u; else c = mid;
@@ -1324,7 +1345,10 @@ __global__ __launch_bounds__(G::NT, 2048 / G::NT) void filter_compact_kernel(Fil
   if (P.top_k > 0) {
     uint32_t cr = 0;
 #pragma unroll
-    for (int i = 0; i < CMAX; ++i) cr += rn[i];
+    for (int i = 0; i < CMAX; ++i) {
+      if (past(i)) break;
+      cr += rn[i];
+    }
     uint32_t tk;
     const uint32_t below = block_excl_scan1<uint32_t, NW>(cr, sh.red_u + 4 * NW, &tk);
     const uint32_t above = tk - below - cr;  // elements of the later (larger) entries
@@ -1352,8 +1376,10 @@ __global__ __launch_bounds__(G::NT, 2048 / G::NT) void filter_compact_kernel(Fil
   // ---- normaliser over the kept-k values ------------------------------------
   double zs[1] = {0.0};
 #pragma unroll
-  for (int i = 0; i < CMAX; ++i)
+  for (int i = 0; i < CMAX; ++i) {
+    if (past(i)) break;
     if (in_k(i)) zs[0] += (double)rn[i] * (double)re[i];
+  }
   block_sum1<double, 1, NW>(zs, sh.red_d);
   const float Z = (float)zs[0];
 
@@ -1365,15 +1391,22 @@ __global__ __launch_bounds__(G::NT, 2048 / G::NT) void filter_compact_kernel(Fil
     auto pmass = [&](uint32_t j) -> double {
       return DEC16 ? (double)round_trip<E>(eat(j) / Z) : (double)(eat(j) * inv);
     };
-    // the share's probabilities (in place of the exponentials, which the
-    // group phase reads from LDS)
-    float* rp = re;
+    // the share's probabilities: 16-bit ones take the place of the exponentials, which
+    // the group phase then reads from LDS; fp32 ones are a product away from them
+    if constexpr (DEC16) {
 #pragma unroll
-    for (int i = 0; i < CMAX; ++i) rp[i] = DEC16 ? round_trip<E>(re[i] / Z) : re[i] * inv;
+      for (int i = 0; i < CMAX; ++i) {
+        if (past(i)) break;
+        re[i] = round_trip<E>(re[i] / Z);
+      }
+    }
+    auto prob = [&](int i) { return (double)(DEC16 ? re[i] : re[i] * inv); };
     double mt = 0.0;
 #pragma unroll
-    for (int i = 0; i < CMAX; ++i)
-      if (in_k(i)) mt += (double)rn[i] * (double)rp[i];
+    for (int i = 0; i < CMAX; ++i) {
+      if (past(i)) break;
+      if (in_k(i)) mt += (double)rn[i] * prob(i);
+    }
     double mtot;
     const double X0 = block_excl_scan1<double, NW>(mt, sh.red_d + NW, &mtot);
     // first addition t in [1, n] of a run X + t p for which hit() holds
@@ -1407,10 +1440,15 @@ __global__ __launch_bounds__(G::NT, 2048 / G::NT) void filter_compact_kernel(Fil
       double X = X0;
       bool found = false;
       uint32_t fk = 0, fp = 0;
+      // only a share whose end may have crossed can hold the crossing (its sum in
+      // another association: a margin of 2^-40); a wave without such a share, or with
+      // nothing left to find, goes on
+      const bool search = hit((X0 + mt) * (1.0 + 0x1p-40));
 #pragma unroll
       for (int i = 0; i < CMAX; ++i) {
-        if (!found && in_k(i)) {
-          const double p = (double)rp[i];
+        if (i % kGroup == 0 && (past(i) || __ballot(search && !found) == 0ull)) break;
+        if (search && !found && in_k(i)) {
+          const double p = prob(i);
           const uint32_t n = rn[i];
           if (hit(X + (double)n * p)) {
             found = true;
@@ -1443,8 +1481,9 @@ __global__ __launch_bounds__(G::NT, 2048 / G::NT) void filter_compact_kernel(Fil
       double bt = 0.0, Xe = X0, smin = INFINITY, hmax = -INFINITY;
 #pragma unroll
       for (int i = 0; i < CMAX; ++i) {
+        if (past(i)) break;
         if (in_k(i)) {
-          const double p = (double)rp[i];
+          const double p = prob(i);
           const uint32_t n = rn[i];
           const double X1 = Xe + (double)n * p;
           bt += run_error_bound(n, p, Xe, X1);
@@ -1469,7 +1508,7 @@ __global__ __launch_bounds__(G::NT, 2048 / G::NT) void filter_compact_kernel(Fil
 #pragma unroll
         for (int i = 0; i < CMAX; ++i) {
           if (!(flo && fhi) && in_k(i)) {
-            const double p = (double)rp[i];
+            const double p = prob(i);
             const uint32_t n = rn[i];
             const uint32_t j = j0 + (uint32_t)i;
             const double X1 = X + (double)n * p;
@@ -1640,14 +1679,17 @@ __global__ __launch_bounds__(G::NT, 2048 / G::NT) void filter_compact_kernel(Fil
   }
   double ksum_above = 0.0;  // kept mass above the group
   uint32_t cnts[3] = {0u, 0u, 0u};  // elements above the group, in it, in it before the cut entry
+  // (a wave whose shares all lie below the group, most of a top-p row, skips the loop)
+  const bool reaches = j1 > g_lo;
 #pragma unroll
   for (int i = 0; i < CMAX; ++i) {
+    if (i % kGroup == 0 && (past(i) || __ballot(reaches) == 0ull)) break;
     const uint32_t j = j0 + (uint32_t)i;
     const uint32_t n = rn[i];
     if (n == 0u) continue;
     if (j > g_hi) {
       cnts[0] += n;
-      ksum_above += (double)n * (double)eat(j);
+      ksum_above += (double)n * (double)(DEC16 && P.has_p ? eat(j) : re[i]);
     } else if (j >= g_lo) {
       cnts[1] += n;
       if (have_cut && j < cut_ent) cnts[2] += n;
@@ -1665,16 +1707,10 @@ __global__ __launch_bounds__(G::NT, 2048 / G::NT) void filter_compact_kernel(Fil
       for (int q = 0; q < 3; ++q) sh.red_u[(5 + q) * NW + wv] = ic[q];
     }
     __syncthreads();
-    ksum_above = 0.0;
+    ksum_above = lane_value(row16_scan(lane < NW ? sh.red_d[3 * NW + lane] : 0.0), NW - 1);
 #pragma unroll
-    for (int w = 0; w < NW; ++w) ksum_above += sh.red_d[3 * NW + w];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      uint32_t sq = 0u;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) sq += sh.red_u[(5 + q) * NW + w];
-      cnts[q] = sq;
-    }
+    for (int q = 0; q < 3; ++q)
+      cnts[q] = lane_value(row16_scan(lane < NW ? sh.red_u[(5 + q) * NW + lane] : 0u), NW - 1);
   }
   double sums[1] = {ksum_above};
   const uint32_t n_group = cnts[1];
