@@ -1048,7 +1048,7 @@ def filtered_bwd(
     logits by it, made before the forward, to the written gradient last (the product
     with ``fl32(1.0 / grad_temperature)`` in the dtype), folded into this write.  ``top_k`` is the forward's; it picks the
     kernel schedule only (rows with kept lists for 1 <= top_k <= 1024).  Rows without
-    kept lists are written in 4 KB pieces with a workspace allocated here (``pieces``;
+    kept lists are written in 8 KB pieces with a workspace allocated here (``pieces``;
     False walks each row with a workgroup of its own: the same gradient)."""
     dev = _require_gpu(logits, target, grad_out, grad_in)
     B, R = target.shape

@@ -1670,7 +1670,7 @@ __global__ __launch_bounds__(kPcThreads) void filter_bwd_piece_kernel(FilterBwdP
 // zeros (a piece whose list overflowed is read again whole, 128 bytes a lane, its
 // ties ranked by a wave scan; with 64 elements a step and a round trip each, the few
 // such pieces of a launch took most of it).  Measured on the top-p backward of bf16
-// [2, 2048, 151936] rows: 130 -> 30 us; [4, 4096, 151936]: 0.17 -> 0.05 ms.  Bound by the
+// [2, 2048, 151936] rows: 130 -> 30 us; [4, 4096, 151936]: 0.17 -> 0.04 ms.  Bound by the
 // latency of a row's dependent loads and of its scattered 2-byte stores.  A decoupled look-back in the piece
 // kernel (each piece adding up the counts its row's earlier pieces publish,
 // so that every tie is written once) measured 2.9 ms for the piece kernel
@@ -1947,7 +1947,7 @@ int launch_bwd(const FilterBwdParams& P, int64_t B, int64_t rows, void* ws, hipS
     if (rows == 0) return MIRL_OK;
     const PieceGeom Gm = piece_geom<E>(P, B, rows, ws);
     if (Gm.ppr > 0) {
-      // 4 KB pieces in address order, then the per-row fix-up of rank-form ties
+      // 8 KB pieces in address order, then the per-row fix-up of rank-form ties
       const int64_t srows = B * P.R;
       auto launch = [&](auto conv) {
         constexpr int CONV = decltype(conv)::value;
