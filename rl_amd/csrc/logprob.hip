@@ -478,7 +478,8 @@ __global__ __launch_bounds__(kFlatThreads) void logprob_bwd_flat_kernel(FlatBwd 
 // aligned vectors, of which one per row may hold the end of that row and the
 // start of the next.  V is at least a piece, so a piece meets at most two rows:
 // both rows' data are uniform (scalar) loads, each lane takes one of them, and
-// the lane whose vector straddles the boundary mixes them element by element.
+// the lane whose vector straddles the boundary mixes them element by element (and
+// loads them so where the second row has no logits: they may end with the first).
 // Elements past the last whole vector are the next lane's.  Same arithmetic as
 // logprob_bwd_flat_kernel.  Measured on [3, 1021, 100003] bf16, 44% of the rows
 // active: 147 us, 6.0 TB/s; the two row-per-workgroup launches 198 us, 4.45 TB/s
@@ -504,6 +505,7 @@ __global__ __launch_bounds__(kFlatThreads) void logprob_bwd_ragged_kernel(FlatBw
     int64_t target;  // flat element of the target, or -1
   };
   RowData d0{0.f, 0.f, 0.f, -1}, d1 = d0;
+  bool whole = false;  // the second row has logits too
   if (A.R > 0) {
     // both rows' loads go out together, from clamped positions
     float gv[2], M[2], LS[2];
@@ -528,6 +530,7 @@ __global__ __launch_bounds__(kFlatThreads) void logprob_bwd_ragged_kernel(FlatBw
     };
     d0 = take(0);
     d1 = take(1);
+    whole = in[1];
   }
   auto grad = [&](float x, const RowData& d, int64_t e) {
     const float p = fast_exp2(((x - d.M) - d.LS) * kLog2e);
@@ -540,7 +543,7 @@ __global__ __launch_bounds__(kFlatThreads) void logprob_bwd_ragged_kernel(FlatBw
     const int64_t i = v0 + threadIdx.x + u * NT, e = i * VEC;
     const bool in0 = e < bound, in1 = e + VEC > bound;
     live[u] = i >= 0 && i < nvec && ((in0 && d0.gv != 0.f) || (in1 && d1.gv != 0.f));
-    if (live[u]) q[u] = __builtin_nontemporal_load(xv + i);
+    if (live[u] && (whole || !(in0 && in1))) q[u] = __builtin_nontemporal_load(xv + i);
   }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -561,11 +564,18 @@ __global__ __launch_bounds__(kFlatThreads) void logprob_bwd_ragged_kernel(FlatBw
       continue;
     }
     float w[VEC], o[VEC];
-    E::unpack(q[u], w);
     if (e < bound && e + VEC > bound) {
+      if (whole) {
+        E::unpack(q[u], w);
+      } else {
+        const raw* x = static_cast<const raw*>(A.logits) + e;
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) w[k] = e + k < bound ? E::load(x + k) : 0.f;
+      }
 #pragma unroll
       for (int k = 0; k < VEC; ++k) o[k] = grad(w[k], e + k < bound ? d0 : d1, e + k);
     } else {
+      E::unpack(q[u], w);
       const bool first = e < bound;
       const float gv = first ? d0.gv : d1.gv, M = first ? d0.M : d1.M, LS = first ? d0.LS : d1.LS;
       const int64_t tj = (first ? d0.target : d1.target) - e;

@@ -39,3 +39,24 @@ def test_flat_pieces_equal_rows(dtype, V, B, S, R):
     own.copy_(x)
     _C.logprob_bwd(own, target, 0, V, stats, up, own)
     assert torch.equal(own, got)
+
+
+@pytest.mark.parametrize("dtype,V", [(torch.bfloat16, 2049), (torch.float16, 6151), (torch.float32, 1027)])
+@pytest.mark.parametrize("B,S,R", [(1, 3, 1), (1, 4, 3), (2, 5, 3)])
+def test_logits_end_with_the_last_row(dtype, V, B, S, R):
+    """Logits that end with row R - 1 of the last sample under a gradient of S > R rows: the
+    vector that holds their end also holds elements of a row without logits."""
+    g = torch.Generator().manual_seed(V + S)
+    flat = (torch.randn((B - 1) * S * V + R * V, generator=g) * 2).to(dtype).to(DEV)
+    x = flat.as_strided((B, R, V), (S * V, V, 1))
+    target = torch.randint(0, V, (B, R), generator=g).to(DEV)
+    target[-1, -1] = V - 1
+    up = torch.randn(B, R, generator=g).to(DEV)
+    stats = torch.empty((B, R, 2), device=DEV)
+    _C.logprob_fwd(x, target, 0, V, torch.empty((B, R), device=DEV), stats)
+    want = torch.empty((B, S, V + 5), dtype=dtype, device=DEV)[..., :V]  # rows of another stride: row kernels
+    _C.logprob_bwd(x, target, 0, V, stats, up, want)
+    got = torch.full((B, S, V), 9.0, dtype=dtype, device=DEV)
+    _C.logprob_bwd(x, target, 0, V, stats, up, got)
+    assert torch.equal(got, want)
+    assert not got[:, R:].any()
