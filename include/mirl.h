@@ -510,9 +510,10 @@ int mirl_gemm_bf16_abt(const void* A, int64_t lda, const void* B, int64_t ldb, i
 /* C = A[:, :K] . B[:, :K]^T in fp32 (A [M, >=K], B [N, >=K] fp32, row strides lda,
  * ldb multiples of 4 elements, 16-byte aligned; K a multiple of 64) on the same
  * MFMA tile loop: each element split into three bf16 planes that add up to it
- * exactly, six products of planes per product, summed in fp32 (tiles with
- * infinities, NaN, values at the top of the range or nonzero values below 2^-109
- * on v_mfma_f32_32x32x2_f32).  C: fp32 [M, ldc] (C = or, with accumulate, C +=),
+ * exactly, the six largest of the nine products of planes per product (the others
+ * are at most 2^-25 of it each), summed in fp32 (tiles with infinities, NaN,
+ * magnitudes or sums from 2^88 on, or nonzero magnitudes of B below 2^-109 on
+ * v_mfma_f32_32x32x2_f32).  C: fp32 [M, ldc] (C = or, with accumulate, C +=),
  * or [k_splits][M][ldc] partial products over k_splits ranges of K (ranges of
  * round_up(ceil(K / k_splits), 64), each non-empty).  `count` as for
  * mirl_gemm_bf16_abt (MIRL_COUNT_ROWS: rows of A at or past *count - count_off

@@ -172,17 +172,11 @@ __device__ __forceinline__ float low_bf16(uint32_t w) {
   return __uint_as_float(__builtin_amdgcn_perm(0u, w, 0x01000c0cu));
 }
 
-// Per 16-bit half of w: 2 w - 1, and the smaller of two.  In asm: taken apart into
-// halves, the compiler converts and permutes each pair again.
-__device__ __forceinline__ uint32_t twice_less_one(uint32_t w) {
-  uint32_t r;
-  asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(r) : "v"(w), "v"(0x00020002u), "v"(0xffffffffu));
-  return r;
-}
-__device__ __forceinline__ uint32_t min_u16x2(uint32_t a, uint32_t b) {
-  uint32_t r;
-  asm("v_pk_min_u16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
+// w | the bits of a and b.  In asm: the compiler would gather the values to join first,
+// on the stack.
+__device__ __forceinline__ uint32_t or3(uint32_t w, float a, float b) {
+  asm("v_or3_b32 %0, %0, %1, %2" : "+v"(w) : "v"(a), "v"(b));
+  return w;
 }
 
 // A value that every lane of the wave holds, in scalar registers.
@@ -535,6 +529,7 @@ void lce_tile_kernel(LceParams P) {
     step(t + 1, S1{}, F_{}, F_{});
   };
 
+  float unscale = 1.f;  // what the accumulators are to be multiplied by (fp32 operands)
   if constexpr (std::is_same<E, F32>::value) {
     // ---- fp32 operands as three bf16 planes each ----
     //
@@ -542,22 +537,31 @@ void lce_tile_kernel(LceParams P) {
     // x2 = x - x0 - x1 (at most eight significant bits are left), so a product of
     // two elements is the sum of nine bf16 products; the three below 2^-25 of it
     // (a1 b2, a2 b1, a2 b2) are left out and the six others summed into the same
-    // fp32 accumulators, the small ones first.  The fp32 MFMA runs at 1/16 of the
-    // bf16 rate, so six bf16 products cost 3/8 of one fp32 product, and 32 k-terms
-    // enter an accumulator in 12 roundings instead of 16: [2048, 4096] x
-    // [65536, 4096]^T 149 -> 237 TFLOP/s (1420 of bf16), error against 64 bits 1.14e-6
-    // -> 1.01e-6 of the result (K = 64: 1.46e-7 -> 1.09e-7).  Bound by the clock: the
+    // fp32 accumulators, the small ones first.  The fp32 MFMA runs at 1/16 of the bf16
+    // rate, so six bf16 products cost 3/8 of one fp32 product, and 32 k-terms enter an
+    // accumulator in 12 roundings instead of 16: [2048, 4096] x [65536, 4096]^T 149 -> 237
+    // TFLOP/s (1420 of bf16), error against 64 bits 1.15e-6 -> 1.00e-6 of the root of the
+    // sum of squared products (K = 64: 1.44e-7 -> 1.09e-7).  Bound by the clock: the
     // MFMA units are busy 87% of the cycles, at 1.5 GHz under this load.
     //
+    // Unscaled, the planes hold all of x from 2^-109 on, and the logits gradient (the
+    // first operand of dH and dW) is less for every improbable token: one such value
+    // sends its tile through both loops below.  So the first operand is multiplied by
+    // 2^40 before it is split and the result by 2^-40: its planes then hold every x below
+    // 2^88, subnormal ones too.  Step of [1024, 2, 4096] x [151936, 4096], every row
+    // active: with logits of standard deviation 10 83.1 -> 50.5 ms, of 1.5 49.4 and 49.3.
+    // (Both operands by 2^24, without the check of the residuals, takes 3% more.)
+    //
     // Each lane reads the fp32 fragments of the coming 16 hidden elements and
-    // splits them while the 96 MFMAs of the current ones run: 52 VALU
-    // instructions per fragment, five in the shadow of each MFMA.  (Residuals by
-    // v_dot2_f32_bf16, 28 instructions, were slower: 207 TFLOP/s.)
+    // splits them while the 96 MFMAs of the current ones run: 56 VALU
+    // instructions per fragment (second operand 48), five or six in the shadow of each
+    // MFMA.  (Residuals by v_dot2_f32_bf16, 28 instructions, were slower: 207 TFLOP/s.)
     using frag16 = typename Mma<BF16>::frag;
+    constexpr float kScale = 0x1p40f, kUnscale = 0x1p-40f;
     constexpr int kPl = 3, kFr = kTM + kTN;
     constexpr int kOpSlots = 11;  // slots a fragment's split takes
     constexpr int kSlots = 2 * kPl * kMB;            // MFMAs per 16 hidden elements
-    constexpr int kOps = 52, kPer = 5;               // VALU ops per fragment, per slot
+    constexpr int kOps = 52, kPer = 5;               // steps of a fragment's split, per slot
     constexpr int kFirst = kSlots - kFr * kOpSlots;  // slot of the first split op
     static_assert(kFirst >= 4 && kKK == 4, "reads ahead of the split");
     // the lane's 8 hidden elements 16 kk + 8 (lane / 32) + 0..7 of a row: two chunks
@@ -569,8 +573,7 @@ void lce_tile_kernel(LceParams P) {
     frag16 pl[2][kFr][kPl];  // [set][A fragments, then B][plane]
     float raw[3][8];
     float h0, h1, r0, r1;
-    // the least nonzero magnitude of a first plane, as 2 |bits| - 1 (zero: 65535)
-    uint32_t mag, least = 0xffffffffu;
+    uint32_t lost = 0;  // the third planes are the last residuals unless one has bits in its low half
     uint32_t out[kPl][4];
     auto read_raw = [&](const unsigned char* stage, int kk, int f) __attribute__((always_inline)) {
       const unsigned char* rows = f < kTM ? stage + (wm * kWM + f * 32) * kRowBytes
@@ -587,19 +590,23 @@ void lce_tile_kernel(LceParams P) {
       constexpr int F = decltype(f_c)::value, N = decltype(n_c)::value;
       constexpr int P = N / 13, O = N % 13;
       float* x = raw[F % 3];
-      if constexpr (O == 0) out[0][P] = BF16::pack2(x[2 * P], x[2 * P + 1]);
-      else if constexpr (O == 1) h0 = low_bf16(out[0][P]);
-      else if constexpr (O == 2) h1 = __uint_as_float(out[0][P] & 0xffff0000u);
-      else if constexpr (O == 3) r0 = x[2 * P] - h0;
-      else if constexpr (O == 4) r1 = x[2 * P + 1] - h1;
-      else if constexpr (O == 5) out[1][P] = BF16::pack2(r0, r1);
-      else if constexpr (O == 6) h0 = low_bf16(out[1][P]);
-      else if constexpr (O == 7) h1 = __uint_as_float(out[1][P] & 0xffff0000u);
-      else if constexpr (O == 8) r0 = r0 - h0;
-      else if constexpr (O == 9) r1 = r1 - h1;
-      else if constexpr (O == 10) out[2][P] = BF16::pack2(r0, r1);
-      else if constexpr (O == 11) mag = twice_less_one(out[0][P]);
-      else least = min_u16x2(least, mag);
+      if constexpr (O == 0) {
+        if constexpr (F < kTM) {
+          x[2 * P] *= kScale;
+          x[2 * P + 1] *= kScale;
+        }
+      } else if constexpr (O == 1) out[0][P] = BF16::pack2(x[2 * P], x[2 * P + 1]);
+      else if constexpr (O == 2) h0 = low_bf16(out[0][P]);
+      else if constexpr (O == 3) h1 = __uint_as_float(out[0][P] & 0xffff0000u);
+      else if constexpr (O == 4) r0 = x[2 * P] - h0;
+      else if constexpr (O == 5) r1 = x[2 * P + 1] - h1;
+      else if constexpr (O == 6) out[1][P] = BF16::pack2(r0, r1);
+      else if constexpr (O == 7) h0 = low_bf16(out[1][P]);
+      else if constexpr (O == 8) h1 = __uint_as_float(out[1][P] & 0xffff0000u);
+      else if constexpr (O == 9) r0 = r0 - h0;
+      else if constexpr (O == 10) r1 = r1 - h1;
+      else if constexpr (O == 11) out[2][P] = BF16::pack2(r0, r1);
+      else lost = or3(lost, r0, r1);
       if constexpr (N == kOps - 1) {
 #pragma unroll
         for (int k = 0; k < kPl; ++k) {
@@ -664,11 +671,10 @@ void lce_tile_kernel(LceParams P) {
       stage2(t + 1, S1{});
     }
     wait_vm_barrier<0>();
-    // Infinities and NaN do not split (inf - inf), a value that rounds up to
-    // infinity does not either, and of values below 2^-109 the last plane falls
-    // under the smallest bf16: a tile in which one shows is formed again with fp32
-    // MFMAs.
-    constexpr uint32_t kLeast = 2u * (18u << 7) - 1u;  // 2^-109
+    // Infinities and NaN do not split (inf - inf), nor does a value that the scale
+    // takes to infinity or that rounds there as a bf16; a sum of 2^88 overflows under
+    // the scale; and a second operand below 2^-109 can have bits that its planes do not
+    // hold: a tile in which one shows is formed again with fp32 MFMAs.
     float z = 0.f;
 #pragma unroll
     for (int i = 0; i < kTM; ++i)
@@ -676,9 +682,11 @@ void lce_tile_kernel(LceParams P) {
       for (int j = 0; j < kTN; ++j)
 #pragma unroll
         for (int v = 0; v < 16; ++v) z += acc[i][j][v] * 0.f;
-    if (__syncthreads_or(!(z == 0.f) || (least & 0xffffu) < kLeast || (least >> 16) < kLeast)) {
+    unscale = kUnscale;
+    if (__syncthreads_or(!(z == 0.f) || (lost & 0xffffu) != 0)) {
       clear_acc();
       run_stages();
+      unscale = 1.f;
     }
   } else {
     run_stages();
@@ -705,7 +713,11 @@ void lce_tile_kernel(LceParams P) {
 #pragma unroll
           for (int g = 0; g < kAV / 4; ++g) {
             const int64_t col = n0 + wn * kWN + j * kT + g * 8 + lane / kT * 4;
-            const f32x4 o = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+            f32x4 o = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+            if constexpr (std::is_same<E, F32>::value) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) o[e] *= unscale;
+            }
             if (col < P.V) put(row, col, o, col + 4 <= P.V);
           }
       }
