@@ -1667,21 +1667,24 @@ __global__ __launch_bounds__(kPcThreads) void filter_bwd_piece_kernel(FilterBwdP
 
 // Per row with a rank-form cut and rcut > 0 (one wave each): the pieces'
 // tie counts scanned in order, and the listed ties of rank < rcut written as
-// zeros (a piece whose list overflowed is read again whole, 128 bytes a lane, its
-// ties ranked by a wave scan; with 64 elements a step and a round trip each, the few
-// such pieces of a launch took most of it).  Measured on the top-p backward of bf16
-// [2, 2048, 151936] rows: 130 -> 30 us; [4, 4096, 151936]: 0.17 -> 0.04 ms.  Bound by the
-// latency of a row's dependent loads and of its scattered 2-byte stores.  A decoupled look-back in the piece
-// kernel (each piece adding up the counts its row's earlier pieces publish,
-// so that every tie is written once) measured 2.9 ms for the piece kernel
-// alone: pieces waiting on pieces of other XCDs hold their slots.
+// zeros (a piece whose list overflowed is read again, 64 bytes a lane in two
+// parts, its ties ranked by a wave scan; with 64 elements a step and a round
+// trip each, the few such pieces of a launch took most of it).  Bound by the
+// latency of a row's dependent loads and of its scattered 2-byte stores, so by the
+// waves in flight: at most 72 registers, seven waves a SIMD (128 bytes a lane in one go
+// took 190 and two).  Measured on the top-p backward of bf16 rows: [2, 2048, 151936]
+// 105 us with the 64-element steps, 24 us with 128 bytes a lane, 19 us now;
+// [2, 16384, 4096], no list overflows, 12.4, 32.0 and 13.6 us.  A decoupled
+// look-back in the piece kernel (each piece adding up the counts its row's earlier
+// pieces publish, so that every tie is written once) measured 2.9 ms for the piece
+// kernel alone: pieces waiting on pieces of other XCDs hold their slots.
 template <class E, int CONV>
-__global__ __launch_bounds__(256) void filter_bwd_piece_fixup_kernel(FilterBwdParams P, PieceGeom Gm,
-                                                                     int64_t nrows) {
+__global__ __launch_bounds__(256, 7) void filter_bwd_piece_fixup_kernel(FilterBwdParams P, PieceGeom Gm,
+                                                                        int64_t nrows) {
   using raw = typename E::raw;
   constexpr int VEC = E::kVec;
-  constexpr int kLV = kPcVectors / 64;  // vectors per lane of a piece read again
-  static_assert(kLV * VEC <= 64, "a lane's ties fit one mask");
+  constexpr int kLV = 4;  // vectors per lane and part of a piece read again
+  static_assert(kLV * VEC <= 32 && kPcVectors % (64 * kLV) == 0, "a lane's ties fit one mask");
   const int lane = threadIdx.x & 63;
   const int64_t srow = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (srow >= nrows) return;
@@ -1730,28 +1733,33 @@ __global__ __launch_bounds__(256) void filter_bwd_piece_fixup_kernel(FilterBwdPa
         rk += (uint32_t)__popcll(bal);
       };
       if (pv == 0) loose(lane, Rw.head);
-      // the body: each lane reads its kLV vectors in one go and ranks its ties
-      // after those of the lanes before it
-      const int i0 = Rw.first(pv) + lane * kLV;
+      // the body in parts of 64 kLV vectors: each lane reads its kLV vectors in one go
+      // and ranks its ties after those of the lanes before it
       const vu4* xv = reinterpret_cast<const vu4*>(x + Rw.head);
-      vu4 q[kLV];
+#pragma unroll 1
+      for (int part = 0; part < kPcVectors; part += 64 * kLV) {
+        const int i0 = Rw.first(pv) + part + lane * kLV;
+        vu4 q[kLV];
 #pragma unroll
-      for (int v = 0; v < kLV; ++v) q[v] = Rw.holds(i0 + v) ? xv[i0 + v] : vu4{0u, 0u, 0u, 0u};
-      uint64_t ties = 0ull;
+        for (int v = 0; v < kLV; ++v) q[v] = Rw.holds(i0 + v) ? xv[i0 + v] : vu4{0u, 0u, 0u, 0u};
+        uint32_t ties = 0u;
 #pragma unroll
-      for (int v = 0; v < kLV; ++v) {
-        float w[VEC];
-        E::unpack(q[v], w);
+        for (int v = 0; v < kLV; ++v) {
+          float w[VEC];
+          E::unpack(q[v], w);
+          uint32_t m = 0u;
 #pragma unroll
-        for (int k = 0; k < VEC; ++k)
-          ties |= (uint64_t)(Rw.holds(i0 + v) && W.yval(w[k]) == W.vc) << (v * VEC + k);
+          for (int k = 0; k < VEC; ++k) m |= (uint32_t)(W.yval(w[k]) == W.vc) << k;
+          ties |= (Rw.holds(i0 + v) ? m : 0u) << (v * VEC);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        const uint32_t nt = (uint32_t)__popc(ties);
+        const uint32_t it = wave_scan_dpp(nt);
+        raw* yb = y + Rw.head + (int64_t)i0 * VEC;
+        for (uint32_t at = rk + it - nt; ties != 0u && at < rcut; ties &= ties - 1u, ++at)
+          yb[__ffs((int)ties) - 1] = zr;
+        rk += (uint32_t)__shfl((int)it, 63, 64);
       }
-      const uint32_t nt = (uint32_t)__popcll(ties);
-      const uint32_t it = wave_scan_dpp(nt);
-      raw* yb = y + Rw.head + (int64_t)i0 * VEC;
-      for (uint32_t at = rk + it - nt; ties != 0ull && at < rcut; ties &= ties - 1ull, ++at)
-        yb[__ffsll((unsigned long long)ties) - 1] = zr;
-      rk += (uint32_t)__shfl((int)it, 63, 64);
       if (pv == Gm.ppr - 1) loose(Rw.tail0 + lane, P.V);
     }
     seen += (uint32_t)__shfl((int)inc, 63, 64);

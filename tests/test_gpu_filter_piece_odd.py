@@ -49,3 +49,24 @@ def test_pieces_equal_walk(dtype, V, tied, T):
         wide = torch.full((B, S, V + 16), 7.0, dtype=dtype, device=DEV)[..., :V]
         _C.filtered_bwd(x, tgt, T, info, kidx, kp, up, wide, top_k=0)
         assert torch.equal(wide, out[0])
+
+
+@pytest.mark.parametrize("dtype,V", [(torch.bfloat16, 4099), (torch.bfloat16, 12290), (torch.float16, 8200),
+                                     (torch.float32, 6149)])
+@pytest.mark.parametrize("p", [0.97, 0.7, 0.45, 0.2])
+def test_rank_cut_in_each_part_of_a_piece(dtype, V, p):
+    """Rows of one value: every list overflows and the cut's rank falls into another part of
+    another piece for each p."""
+    B, S = 1, 9
+    x = torch.zeros(B, S, V, dtype=dtype, device=DEV)
+    tgt = torch.full((B, S - 1), V - 1, dtype=torch.int64, device=DEV)
+    up = torch.ones(B, S - 1, device=DEV)
+    info, kidx, kp = _C.filtered_fwd(x, tgt, 1.0, 0, p, None, torch.float32 if dtype != torch.float32 else None)
+    out = []
+    for pieces in (True, False):
+        grad = torch.full((B, S, V), 7.0, dtype=dtype, device=DEV)
+        _C.filtered_bwd(x, tgt, 1.0, info, kidx, kp, up, grad, top_k=0, pieces=pieces)
+        out.append(grad)
+    assert torch.equal(out[0], out[1])
+    kept = (out[0][0, :-1] != 0).sum(-1)
+    assert (kept >= int(p * V) - 8).all() and (kept <= int(p * V) + 8).all()
