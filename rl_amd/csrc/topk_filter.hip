@@ -1452,26 +1452,28 @@ static_assert(kPieceTieCap % 2 == 0, "a piece's list is read as 32-bit words");
 
 struct PieceGeom {
   int ppr;            // pieces per row (the most that a row of V elements can have)
+  int skew_mask;      // kPcLine - 1: pieces start on 128-byte lines; 0: on the row's first vector
   uint32_t* tie_cnt;  // [B * R * ppr]: the piece's tie count (rank-form rows with rcut > 0)
   uint16_t* tie_pos;  // [B * R * ppr][kPieceTieCap]: tie offsets from the piece's first element
 };
 
 // A row's elements before its first 16-byte vector, its vectors, and the first element
 // after them.  They differ from row to row where V is not a multiple of a vector.  Pieces
-// start on 128-byte lines: the first one `skew` vectors before the row's first, so that
-// no line but a row's first and last is written by two workgroups.  The last piece may be
-// without any vector and still write the elements after them.
+// start on 128-byte lines (unless pieces_of says otherwise): the first one `skew` vectors
+// before the row's first, so that no line but a row's first and last is written by two
+// workgroups.  The last piece may be without any vector and still write the elements
+// after them.
 template <class E>
 struct PieceRow {
   int head, nvec, tail0, skew;
-  __device__ __forceinline__ PieceRow(const typename E::raw* y, int64_t V) {
+  __device__ __forceinline__ PieceRow(const typename E::raw* y, int64_t V, int skew_mask) {
     // (RowSpan in 32 bits, V < 2^31: a piece is short enough for scalar work to show)
     const uint32_t v = (uint32_t)V, vec = E::kVec;
     const uint32_t h = min((0u - (uint32_t)reinterpret_cast<uintptr_t>(y) & 15u) / (16u / vec), v);
     head = (int)h;
     nvec = (int)((v - h) / vec);
     tail0 = head + nvec * (int)vec;
-    skew = (int)(reinterpret_cast<uintptr_t>(y + head) >> 4) & (kPcLine - 1);
+    skew = (int)(reinterpret_cast<uintptr_t>(y + head) >> 4) & skew_mask;
   }
   // the vector at which piece pc starts
   __device__ __forceinline__ int first(int pc) const { return pc * kPcVectors - skew; }
@@ -1505,7 +1507,7 @@ __global__ __launch_bounds__(kPcThreads) void filter_bwd_piece_kernel(FilterBwdP
     t = P.target[(int64_t)b * P.tsb + (int64_t)r * P.tsr];
   }
   raw* y = static_cast<raw*>(P.gin) + (int64_t)b * P.gisb + (int64_t)r * P.gisr;
-  const PieceRow<E> Rw(y, P.V);
+  const PieceRow<E> Rw(y, P.V, Gm.skew_mask);
   vu4* yv = reinterpret_cast<vu4*>(y + Rw.head);
   const int i0 = Rw.first(pc) + tid;  // this thread's first vector
   const int tail0 = Rw.tail0;
@@ -1696,7 +1698,7 @@ __global__ __launch_bounds__(256, 7) void filter_bwd_piece_fixup_kernel(FilterBw
   const uint32_t rcut = (uint32_t)(-1 - ri.i_cut);
   raw* y = static_cast<raw*>(P.gin) + b * P.gisb + r * P.gisr;
   const raw* x = static_cast<const raw*>(P.logits) + b * P.sb + r * P.sr;
-  const PieceRow<E> Rw(y, P.V);
+  const PieceRow<E> Rw(y, P.V, Gm.skew_mask);
   const raw zr = E::from_float(0.f);
   const WalkMath<E, CONV> W(P, ri, gv, -1);
   const uint32_t* cnt = Gm.tie_cnt + srow * Gm.ppr;
@@ -1913,11 +1915,22 @@ int launch_topk_export(const FilterParams& P, int64_t rows, hipStream_t st) {
   return check_launch("topk_export_general_kernel");
 }
 
-// The most pieces that a row of V elements can have, whatever line its first vector starts in.
-int64_t piece_ppr_bound(int64_t V, int64_t esz) {
-  const int64_t nv = V * esz / 16;
-  return nv > 0 ? (nv + kPcLine - 1 + kPcVectors - 1) / kPcVectors : 1;
+// Pieces of a row of nv vectors whose first piece may start `skew` vectors ahead of it, on a
+// 128-byte line (*lines: whether it does).  Where that takes one piece more, almost empty,
+// 16-bit rows start on their own first vector and share lines between workgroups: backward
+// of bf16 [2, 16384, 4088] 103 us, 171 on lines; [2, 4578, 32760] 203 and 215;
+// [2, 1144, 131064] 202 and 205.  fp32 pieces hold half the values and cost less than
+// shared lines from two pieces on: [2, 9159, 8188] 198 us, 192 on lines; [2, 1144, 65532]
+// 195 and 189; one piece alone [2, 16384, 2044] 93 and 113.
+int64_t pieces_of(int64_t nv, int64_t skew, int64_t esz, bool* lines = nullptr) {
+  const int64_t n = std::max<int64_t>(1, (nv + kPcVectors - 1) / kPcVectors);
+  const int64_t on_lines = std::max<int64_t>(1, (nv + skew + kPcVectors - 1) / kPcVectors);
+  const bool l = on_lines == n || (esz == 4 && n >= 2);
+  if (lines != nullptr) *lines = l;
+  return l ? on_lines : n;
 }
+// The most pieces that a row of V elements is cut into, whatever line its first vector is in.
+int64_t piece_ppr_bound(int64_t V, int64_t esz) { return pieces_of(V * esz / 16, kPcLine - 1, esz); }
 
 // The piece schedule's geometry when the layout allows it (each row of the logits and
 // its gradient at the same offset from a 16-byte boundary, rows whole in 32-bit
@@ -1931,14 +1944,17 @@ PieceGeom piece_geom(const FilterBwdParams& P, int64_t B, int64_t rows, void* ws
   if (ws == nullptr || ax % esz != 0 || ay % esz != 0) return Gm;
   // without rows to read (R = 0) the logits' place does not matter
   if (P.R > 0 && (ax % 16 != ay % 16 || !steps_ok(P.sb, P.gisb, B) || !steps_ok(P.sr, P.gisr, P.R))) return Gm;
-  int64_t ppr = piece_ppr_bound(P.V, esz);
+  // vectors of a row, and those by which its first piece may start ahead: the most of any
+  // row, or what they are where every row starts at the same place of a line
+  int64_t nvec = P.V * esz / 16, skew = kPcLine - 1;
   if ((B <= 1 || P.gisb * esz % 128 == 0) && (P.Rt <= 1 || P.gisr * esz % 128 == 0)) {
-    // every row starts at the same place of a line: no piece more than they need
-    // (131072 elements in 32 pieces: an empty 33rd cost the kernel 6%)
-    const int64_t head = std::min<int64_t>((16 - ay % 16) % 16 / esz, P.V), nvec = (P.V - head) / E::kVec;
-    const int64_t skew = (int64_t)(ay / 16 + (ay % 16 != 0)) % kPcLine;
-    ppr = std::max<int64_t>(1, (nvec + skew + kPcVectors - 1) / kPcVectors);
+    const int64_t head = std::min<int64_t>((16 - ay % 16) % 16 / esz, P.V);
+    nvec = (P.V - head) / E::kVec;
+    skew = (int64_t)(ay / 16 + (ay % 16 != 0)) % kPcLine;
   }
+  bool lines;
+  const int64_t ppr = pieces_of(nvec, skew, esz, &lines);
+  Gm.skew_mask = lines ? kPcLine - 1 : 0;
   if (rows * ppr * kPcThreads >= (int64_t(1) << 32)) return Gm;
   // workspace: the tie counts, then the tie lists
   const int64_t slots = B * P.R * ppr;

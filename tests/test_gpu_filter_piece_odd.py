@@ -17,7 +17,9 @@ DEV = torch.device("cuda", 0)
 @pytest.mark.parametrize("dtype,V", [(torch.bfloat16, 5), (torch.bfloat16, 13), (torch.bfloat16, 4095),
                                      (torch.bfloat16, 4099), (torch.bfloat16, 4105), (torch.bfloat16, 4107),
                                      (torch.bfloat16, 38931), (torch.float16, 4107), (torch.float32, 2047),
-                                     (torch.float32, 2053), (torch.float32, 20002)])
+                                     (torch.float32, 2053), (torch.float32, 20002),
+                                     # whole vectors: pieces on lines would be one more
+                                     (torch.bfloat16, 4088), (torch.float16, 8184), (torch.float32, 2044)])
 @pytest.mark.parametrize("tied", [1, 8, 400])  # elements per distinct value: listed ties, and lists that overflow
 @pytest.mark.parametrize("T", [1.0, 0.7])
 def test_pieces_equal_walk(dtype, V, tied, T):

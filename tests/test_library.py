@@ -105,3 +105,17 @@ def test_binding_argument_types_follow_the_header():
             if not _ctype_matches(pt, ct):
                 bad.append((name, k, pt, ct))
     assert not bad, bad
+
+
+@pytest.mark.parametrize("name,V", [("bfloat16", 4088), ("bfloat16", 8184), ("float16", 8191), ("bfloat16", 131064),
+                                    ("bfloat16", 151936), ("float32", 2044), ("bfloat16", 5)])
+def test_filtered_backward_cuts_rows_into_no_spare_piece(name, V):
+    """The filtered backward's workspace holds as many 8 KB pieces as a row's vectors fill, for
+    rows that start anywhere in a 128-byte line (512 vectors a piece, 4 + 2 * 14 bytes each)."""
+    import torch
+
+    from rl_amd import _C
+
+    code = _C.DTYPE_CODES[getattr(torch, name)]
+    pieces = max(1, -(-(V // (4 if name == "float32" else 8)) // 512))
+    assert _C.load().mirl_filtered_logprob_bwd_workspace_bytes(code, 3, 5, V) == 3 * 5 * pieces * 32
