@@ -868,10 +868,18 @@ def divergence_bwd(
 # ---------------------------------------------------------------------------
 # GRPO advantages
 # ---------------------------------------------------------------------------
-# Up to this many prompt rows are compared pair by pair in one launch; more are hashed
-# first, in two more launches: 16 rows of 512 tokens take 11 us directly and 16 us hashed,
-# 32 rows 20 and 16 us, 64 rows 37 and 16 us.
-_ADV_DIRECT_ROWS = 16
+# Prompt rows are compared pair by pair in one launch while that takes less than the 14.5 us
+# that the host needs for the three launches of the hashed path (8-13 us on the GPU, 26 for
+# 16384 tokens).  A pair that shares its first token costs a wave 0.23 us and 0.85 us per 1024
+# tokens, so the line lies at a number of rows times 1 + K / 256.  Rows of K tokens, us
+# directly and hashed: K = 64: 24 rows 9.9 / 14.5, 64 rows 20.0 / 14.6; K = 512: 16 rows
+# 11.5 / 14, 24 rows 16.1 / 14.5; K = 4096: 3 rows 9.7 / 14, 8 rows 29 / 14, 16 rows 57 / 15.
+_ADV_DIRECT_ROWS = 52
+
+
+def _adv_direct(B: int, K: int) -> bool:
+    """Whether B prompt rows of K elements are compared pair by pair."""
+    return K == 1 or B <= 2 or B * (256 + K) <= 256 * _ADV_DIRECT_ROWS
 
 
 def grpo_advantage(
@@ -901,7 +909,7 @@ def grpo_advantage(
         int(bool(leave_one_out)), int(bool(normalize)), adv.data_ptr(), _ptr(base), _ptr(std),
         _ptr(trivial),
     )
-    if K > 1 and B > _ADV_DIRECT_ROWS:
+    if not _adv_direct(B, K):
         ws = torch.empty(load().mirl_grpo_advantage_workspace_bytes(B, K), dtype=torch.uint8, device=dev)
         name = "mirl_grpo_advantage_ws"
         st = _launch(name, dev, *args, ws.data_ptr(), _stream(dev))

@@ -162,7 +162,8 @@ __global__ __launch_bounds__(256) void adv_scalar_kernel(AdvArgs A, const T* __r
 
 // Prompt rows compared directly (no workspace).  Each row that agrees in its first
 // element costs a dependent round trip per 64 x 4 elements: 7 us for 8 rows of 512
-// tokens, 11 us for 16, 20 us for 32, against 13-16 us for the three hashed launches.
+// tokens, 11 us for 16, 20 us for 32, 57 us for 16 of 4096, against 13-16 us for the three
+// hashed launches.
 __global__ __launch_bounds__(256) void adv_rows_kernel(AdvArgs A) {
   const int64_t i = wave_sample();
   if (i >= A.B) return;
