@@ -29,6 +29,7 @@
 //
 // The MFMA lane layouts (checked on gfx950) stand at Mma<E>.
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -1155,26 +1156,29 @@ __global__ __launch_bounds__(kActThreads) void lce_active_rows_kernel(
 
 // Row m of the permuted targets and statistics and, for m < *count, of the permuted
 // hidden states (row_units units of UNIT per row; rows past the count stay as they
-// are: every kernel stops at the count).  One workgroup per row.
+// are: every kernel stops at the count).  One workgroup per row, up to kGatherGrid of
+// them: a launch holds fewer than 2^32 threads.
+constexpr int64_t kGatherGrid = int64_t(1) << 20;
 template <class UNIT>
 __global__ __launch_bounds__(256) void lce_gather_rows_kernel(
-    const int64_t* __restrict__ perm, const int64_t* __restrict__ count, uint32_t bsz,
+    const int64_t* __restrict__ perm, const int64_t* __restrict__ count, int64_t T, uint32_t bsz,
     const int64_t* __restrict__ target, int64_t tsb, int64_t tss, const float* __restrict__ stats,
     const UNIT* __restrict__ hidden, int64_t row_units, int64_t ld_units, int64_t* __restrict__ tgt_a,
     float* __restrict__ st_a, UNIT* __restrict__ h_a) {
-  const int64_t m = blockIdx.x;
-  const uint32_t r = (uint32_t)perm[m];
-  const bool live = m < *count;
-  if (threadIdx.x == 0) {
-    const uint32_t s = r / bsz, b = r - s * bsz;
-    tgt_a[m] = target[(int64_t)b * tsb + (int64_t)s * tss];
-    st_a[2 * m] = stats[2 * (int64_t)r];
-    st_a[2 * m + 1] = stats[2 * (int64_t)r + 1];
+  for (int64_t m = blockIdx.x; m < T; m += kGatherGrid) {
+    const uint32_t r = (uint32_t)perm[m];
+    const bool live = m < *count;
+    if (threadIdx.x == 0) {
+      const uint32_t s = r / bsz, b = r - s * bsz;
+      tgt_a[m] = target[(int64_t)b * tsb + (int64_t)s * tss];
+      st_a[2 * m] = stats[2 * (int64_t)r];
+      st_a[2 * m + 1] = stats[2 * (int64_t)r + 1];
+    }
+    if (!live) continue;
+    const UNIT* src = hidden + (int64_t)r * ld_units;
+    UNIT* dst = h_a + m * row_units;
+    for (int64_t k = threadIdx.x; k < row_units; k += 256) dst[k] = src[k];
   }
-  if (!live) return;
-  const UNIT* src = hidden + (int64_t)r * ld_units;
-  UNIT* dst = h_a + m * row_units;
-  for (int64_t k = threadIdx.x; k < row_units; k += 256) dst[k] = src[k];
 }
 
 // Per row: combine the column-tile partials into the row's max and log-sum-exp,
@@ -1569,8 +1573,8 @@ extern "C" int mirl_lce_active_rows(const float* grad_out, int64_t g_stride_b, i
     auto launch = [&](auto unit) {
       using UNIT = decltype(unit);
       constexpr int64_t n = sizeof(UNIT);
-      hipLaunchKernelGGL(lce_gather_rows_kernel<UNIT>, dim3((unsigned)T), dim3(256), 0, st, perm, count,
-                         (uint32_t)bsz, target, t_stride_b, t_stride_s, row_stats,
+      hipLaunchKernelGGL(lce_gather_rows_kernel<UNIT>, dim3((unsigned)std::min(T, kGatherGrid)), dim3(256), 0,
+                         st, perm, count, T, (uint32_t)bsz, target, t_stride_b, t_stride_s, row_stats,
                          static_cast<const UNIT*>(hidden), Hd * esz / n, ldh * esz / n, target_out,
                          stats_out, static_cast<UNIT*>(hidden_out));
     };

@@ -35,3 +35,21 @@ def test_active_rows(S, B, H, pad, dtype, share):
     assert torch.equal(h[:n], wide[:, :H][active])
     assert torch.equal(tgt[0], target.t().reshape(T)[perm]) and torch.equal(st, stats[perm])
     torch.testing.assert_close(ga[0], rows[perm], rtol=0, atol=0, equal_nan=True)
+
+
+@pytest.mark.parametrize("T", [(1 << 20) + 5, (1 << 24) + 5])
+def test_more_rows_than_a_launch_holds_workgroups_for(T):
+    """2^24 rows of 256 threads each would be 2^32 threads, more than a launch takes."""
+    g = torch.Generator(device=DEV).manual_seed(T)
+    up = torch.randn(1, T, generator=g, device=DEV) * (torch.rand(1, T, generator=g, device=DEV) < 0.5)
+    target = torch.randint(0, 1000, (1, T), generator=g, device=DEV)
+    stats = torch.randn(T, 2, generator=g, device=DEV)
+    hidden = torch.randn(T, 8, generator=g, device=DEV).to(torch.bfloat16)
+    perm, count, h, tgt, st, ga = _C.lce_active_rows(up, target, stats, hidden)
+    active = (up[0] != 0).nonzero()[:, 0]
+    n = int(count)
+    assert n == active.numel()
+    assert torch.equal(perm[:n], active)
+    assert torch.equal(perm[n:], (up[0] == 0).nonzero()[:, 0].flip(0))
+    assert torch.equal(h[:n], hidden[active])
+    assert torch.equal(tgt[0], target[0][perm]) and torch.equal(st, stats[perm]) and torch.equal(ga[0], up[0][perm])
