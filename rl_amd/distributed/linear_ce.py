@@ -380,6 +380,7 @@ def _f32_backward(ctx, grad_output):
 _FUSED_DTYPES = (torch.bfloat16, torch.float16)  # operand dtypes of the fused kernels
 _F32_K_ALIGN = 64  # the fp32 tile loop steps through the reduction 64 elements at a time
 _BLOCK_CHUNKS = 4  # chunks of active rows per backward block
+_BLOCK_TILES = 512  # 256 x 256 tiles of the logits that a block has at least: two per CU
 _K_ALIGN = 128  # dW's reduction length is padded with zero rows to a multiple of this
 _H_ALIGN = 128  # the fused kernels step through the hidden dimension 128 elements at a time
 
@@ -415,7 +416,7 @@ def _block_rows(T: int, chunk_size: Optional[int], rows_per_position: int, V: in
     and one 256-row strip of the logits."""
     if chunk_size is None:
         return T
-    least = 256 * -(-512 // -(-V // 256))
+    least = 256 * -(-_BLOCK_TILES // -(-V // 256))
     return min(T, max(_round_up(chunk_size * rows_per_position, 256), least))
 
 

@@ -21,6 +21,7 @@ from oracle.linear_ce import (
     logits_bf16,
     next_token_hidden_state_logprobs,
 )
+from rl_amd.distributed import linear_ce
 from rl_amd.distributed.model_utils import (
     ChunkedDistributedHiddenStatesToLogprobs,
     from_parallel_hidden_states_to_logprobs,
@@ -249,27 +250,40 @@ def test_fp16_fp32_forward_and_gradients(dtype, S, B, H, V, chunk):
         assert err <= rel * want.abs().max().item(), (err, want.abs().max().item())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("inline", [True, False])
 @pytest.mark.parametrize("active", [0.0, 0.2, 0.6, 1.0])
-def test_gradient_blocks_with_device_count(active):
-    """Several backward blocks (600 rows, 256 per block at chunk 7): the active-row count
+def test_gradient_blocks_with_device_count(active, inline, dtype, monkeypatch):
+    """Several backward blocks (600 rows, 256 per block at chunk 7 without the rows that a small
+    vocabulary adds to a block; in fp32 of the forward too): the active-row count
     lives on the device, so the blocks past it return at once and dW is rounded by the
-    last block holding active rows (none, the first, the second, the third)."""
-    say("linear-ce grad blocks active", active)
+    last block holding active rows (none, the first, the second, the third).  W^T formed on
+    the current stream (inline) and, as a large weight's is, on the side stream."""
+    say("linear-ce grad blocks active", active, inline, dtype)
     S, B, H, V = 200, 3, 128, 2000
-    hidden, weight, target = _inputs(S, B, H, V, seed=61)
+    monkeypatch.setattr(linear_ce, "_BLOCK_TILES", 1)
+    if not inline:
+        monkeypatch.setattr(linear_ce, "_INLINE_TRANSPOSE", 0)
+    per = B if dtype == torch.float32 else linear_ce._BLOCK_CHUNKS * B
+    assert linear_ce._block_rows(S * B, 7, per, V) == 256  # three blocks
+    hidden, weight, target = (x if x.dtype == torch.int64 else x.to(dtype) for x in _inputs(S, B, H, V, seed=61))
     gen = torch.Generator().manual_seed(62)
     g = torch.randn(B, S, generator=gen) * (torch.rand(B, S, generator=gen) < active).float()
     h = hidden.to(DEV).requires_grad_(True)
     w = weight.to(DEV).requires_grad_(True)
     lp = ChunkedDistributedHiddenStatesToLogprobs.apply(h, target.to(DEV), w, 0, V, 7, None, False)
+    if dtype == torch.float32:
+        ref = hidden_state_logprobs(hidden, target, weight, 0, V)
+        assert (lp.detach().cpu().double() - ref.double()).abs().max().item() < 1e-4
     dh, dw = torch.autograd.grad(lp, [h, w], g.to(DEV))
     if active == 0.0:
         assert not dh.any() and not dw.any()
         return
     rdh, rdw, _ = hidden_state_logprob_grads(hidden, target, weight, 0, V, g)
+    rel = 1e-4 if dtype == torch.float32 else 1e-2
     for got, ref in ((dh, rdh), (dw, rdw)):
         err = (got.cpu().double() - ref).abs().max().item()
-        assert err <= 1e-2 * ref.abs().max().item(), (active, err)
+        assert err <= rel * ref.abs().max().item(), (active, err)
     assert not dh.cpu()[(g == 0).t()].any()
 
 
@@ -483,11 +497,15 @@ def test_f32_path_runs_no_library_gemm(monkeypatch):
         assert (got.cpu().double() - want).abs().max().item() <= 1e-4 * want.abs().max().item()
 
 
-def test_weight_written_in_place_between_backwards():
+@pytest.mark.parametrize("inline", [True, False])
+def test_weight_written_in_place_between_backwards(inline, monkeypatch):
     """A weight changed without its version counter moving (``p.data.copy_``, as Megatron
     and collectives write parameters) gives the next backward the new weight: dH and dW
-    equal, bit for bit, those of a fresh weight tensor holding the same values."""
-    say("linear-ce weight written in place")
+    equal, bit for bit, those of a fresh weight tensor holding the same values.  W^T on the
+    current stream (inline) and on the side stream of large weights."""
+    say("linear-ce weight written in place", inline)
+    if not inline:
+        monkeypatch.setattr(linear_ce, "_INLINE_TRANSPOSE", 0)
     S, B, H, V = 40, 2, 256, 3001
     hidden, weight, target = _inputs(S, B, H, V, seed=51)
     _, weight2, _ = _inputs(S, B, H, V, seed=52)
