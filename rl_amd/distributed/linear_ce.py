@@ -145,9 +145,9 @@ class ChunkedDistributedHiddenStatesToLogprobs(torch.autograd.Function):
         # order) and their count stays on the device: every kernel below reads it
         # and skips what lies past it, so the host never waits for the count.
         perm, count, h_a, tgt_a, st_a, g_a = _C.lce_active_rows(grad_output, target, stats, h2)
-        # Blocks of up to 4 chunks of rows (whole 256-row tiles): the bf16 G
-        # buffer stays below one reference chunk's fp32 logits, softmax and
-        # one-hot temporaries.  Blocks past the count return at once.
+        # Blocks of 4 chunks of rows (whole 256-row tiles; the bf16 G then stays below
+        # one reference chunk's fp32 logits, softmax and one-hot temporaries), or of the
+        # rows that fill the chip.  Blocks past the count return at once.
         rows = _block_rows(T, ctx.chunk_size, _BLOCK_CHUNKS * B, V)
         n_blocks = -(-T // rows)
         Vp = _round_up(V, _K_ALIGN)
@@ -320,10 +320,11 @@ def _f32_forward(ctx, hidden, target, weight, vs, ve, chunk_size, inference_only
 def _f32_backward(ctx, grad_output):
     """fp32 backward (reference model_utils.py:2647-2745) over the rows with a non-zero
     upstream gradient, moved to the front and counted on the device (the others have a zero
-    logits gradient: zero dH rows, nothing added to dW).  Per block of one chunk of rows:
-    the logits recomputed on the fp32 tile loop, G = (onehot - softmax) * g written over them
-    by the logprob backward kernel, dH = G . W against W^T, and dW += G^T . H, fp32
-    throughout."""
+    logits gradient: zero dH rows, nothing added to dW).  Per block of at least one chunk of
+    rows: the logits recomputed on the fp32 tile loop, G = (onehot - softmax) * g written over
+    them by the logprob backward kernel, dH = G . W against W^T, and dW += G^T . H, with fp32
+    operands, sums and results (the loop forms a product of two fp32 values from six of the
+    nine products of their bf16 planes)."""
     hidden, target, weight, stats = ctx.saved_tensors
     vs, ve = ctx.vocab
     S, B, H = hidden.shape
@@ -412,8 +413,14 @@ def _block_rows(T: int, chunk_size: Optional[int], rows_per_position: int, V: in
     (``rows_per_position`` rows a position) in whole 256-row tiles, and at least as many as
     give every CU two 256 x 256 tiles of the [rows, V] logits.  Fewer leave CUs idle and
     tiles partly empty (64-row chunks of [512, 1024] x [32000, 1024] fp32: 2.2 ms of kernels;
-    the whole step takes 0.62 ms in one block); the scratch this adds is at most 512 such tiles (134 MB in fp32)
-    and one 256-row strip of the logits."""
+    the whole step takes 0.62 ms in one block).
+
+    What these rows add to a block's scratch: [rows, V] arrays of 512 tiles and one 256-row
+    strip of the logits (fp32: 134 MB and 1 KB per vocabulary entry), one in the fp32 forward,
+    two in a backward (G and its transpose), and dH's partial products, [splits, rows, H] fp32:
+    at most 64 MiB where these have fewer than 32 tiles, else ceil(V / 1024) times [rows, H]
+    (fp32, V = 4000, H = 4096: 8192 rows, G and its transpose 131 MB each and 268 MB of
+    partials, beside the [T, H] copies that every backward holds)."""
     if chunk_size is None:
         return T
     least = 256 * -(-_BLOCK_TILES // -(-V // 256))

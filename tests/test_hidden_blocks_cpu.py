@@ -29,3 +29,17 @@ def test_blocks_hold_a_chunk_and_fill_the_chip(T, chunk, per, V):
     if chunk is not None:
         # beyond a chunk: at most 512 tiles and one strip of the logits
         assert rows <= -(-chunk * per // 256) * 256 or rows * V <= 512 * 256 * 256 + 256 * V
+
+
+@pytest.mark.parametrize("V", [300, 1000, 2047, 4000, 9973, 32000, 151936])
+@pytest.mark.parametrize("H", [64, 1024, 4096, 8192])
+def test_scratch_of_a_block(V, H):
+    """The fp32 backward's scratch for a block of a tiny chunk: logits, their transpose and dH's
+    partial products stay within what _block_rows states."""
+    rows = _block_rows(1 << 24, 1, 1, V)
+    K = -(-V // 64) * 64
+    part = _dh_splits(rows, H, K, count_known=False) * rows * H
+    assert rows * V <= 512 * 65536 + 256 * V
+    assert part <= max(1 << 24, -(-V // 1024) * rows * H)
+    if (V, H) == (4000, 4096):
+        assert rows == 8192 and part * 4 == 268435456
