@@ -540,10 +540,12 @@ void lce_tile_kernel(LceParams P) {
     // (a1 b2, a2 b1, a2 b2) are left out and the six others summed into the same
     // fp32 accumulators, the small ones first.  The fp32 MFMA runs at 1/16 of the bf16
     // rate, so six bf16 products cost 3/8 of one fp32 product, and 32 k-terms enter an
-    // accumulator in 12 roundings instead of 16: [2048, 4096] x [65536, 4096]^T 149 -> 237
-    // TFLOP/s (1420 of bf16), error against 64 bits 1.15e-6 -> 1.00e-6 of the root of the
-    // sum of squared products (K = 64: 1.44e-7 -> 1.09e-7).  Bound by the clock: the
-    // MFMA units are busy 87% of the cycles, at 1.5 GHz under this load.
+    // accumulator in 12 roundings instead of 16: [2048, 4096] x [65536, 4096]^T 151 -> 241
+    // TFLOP/s back to back (1450 of bf16), error against 64 bits 1.15e-6 -> 1.00e-6 of the root
+    // of the sum of squared products (K = 64: 1.44e-7 -> 1.10e-7; sums of two terms 3.1e-8
+    // -> 3.3e-8, of one 2.5e-8 -> 3.4e-8: what is left out counts there).  Bound by the MFMA
+    // units, busy 87% of the cycles at the 1.5 GHz that this load leaves (82% at 1.92 GHz
+    // and 276 TFLOP/s where memory-bound kernels run in between).
     //
     // Unscaled, the planes hold all of x from 2^-109 on, and the logits gradient (the
     // first operand of dH and dW) is less for every improbable token: one such value

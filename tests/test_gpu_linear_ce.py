@@ -216,8 +216,8 @@ def test_gradient_row_compaction(pattern):
 @pytest.mark.parametrize("S,B,H,V,chunk", [(37, 3, 128, 1000, 8), (16, 2, 64, 151936, None), (9, 3, 200, 3001, 4)])
 def test_fp16_fp32_forward_and_gradients(dtype, S, B, H, V, chunk):
     """fp16 inputs run the fused kernels (logits tiles on the fp16 MFMA, rounded to fp16;
-    G in bf16 and W, H rounded to bf16 for dH and dW); fp32 inputs take per chunk the fp32
-    tile loop (fp32 MFMA), then the logprob row kernels (the reference's chunked shape), and
+    G in bf16 and W, H rounded to bf16 for dH and dW); fp32 inputs take per block the fp32
+    tile loop (bf16 planes), then the logprob row kernels (the reference's chunked shape), and
     the backward's three products on the fp32 tile loop over the active rows.  The oracle
     rounds the exact products to the dtype; logprobs within 2e-3 (fp16) / 1e-5 (fp32) plus
     the target logit's last-ulp rounding, dH and dW against the float64 oracle to 1e-2
@@ -404,7 +404,7 @@ def test_gemm_primitives_with_device_counts():
 
 
 def test_gemm_f32_primitives():
-    """The fp32 tile loop (four v_mfma_f32_32x32x2_f32 per fragment pair): C = A . B^T
+    """The fp32 tile loop (six products of bf16 planes per product): C = A . B^T
     against float64 within fp32 summation error; k splits sum to the same product; with a
     device row count absent rows are untouched and the others equal the uncounted call bit
     for bit; a reduction-length count over blocks accumulated in fp32 equals the
